@@ -28,6 +28,9 @@
 #include "lulesh_mesh.hpp"
 
 #include "lulesh_elem.hpp"
+#ifdef LULESH_FUSED
+#include "lulesh_modal.hpp"
+#endif
 
 // FMA contraction off: every value rounded as the reference rounds it;
 // the fused build (LULESH_FUSED) lets multiply-adds fuse
@@ -49,6 +52,291 @@ constexpr int kStencil[8][6] = {{1, 2, 3, 4, 5, 7}, {2, 3, 0, 5, 6, 4},
                                 {7, 6, 5, 0, 3, 1}, {4, 7, 6, 1, 0, 2},
                                 {5, 4, 7, 2, 1, 3}, {6, 5, 4, 3, 2, 0}};
 
+#ifdef LULESH_FUSED
+// The fused build's share of a block: the tile, the halo and the node update
+// of the exact build's sweep_tile, with the element's forces formed in its
+// modes (lulesh_modal.hpp).
+//
+// FP64 issue bounded the corner form (81.5 M VALU wave instructions, 230 us
+// at 150^3); the modal form issues 45.8 M and takes 152 us, now bounded by
+// its two waves per SIMD (244 VGPRs) waiting for each other and for LDS:
+// issue is 57% busy, and its 580 MB pass at 3.8 TB/s of the 5.7 a copy
+// reaches.  What makes up the rest of the difference:
+//  - The forces on the four corners of a face add up over the two layers
+//    that share it before they leave the thread, as face modes (`top`), so a
+//    thread stages three corners per plane for its three neighbours (18 KB)
+//    instead of eight corners twice per layer (48 KB).
+//  - The positions' face modes of the low plane are those of the layer
+//    below's high plane, kept in registers (the velocities' as well would
+//    spill).
+//  - The LDS this frees holds the next plane and the next layer's corners
+//    beside the current ones: one barrier per layer (two: 157 us).
+template <int TX, int TY, class Fields>
+__device__ __forceinline__ void sweep_tile(const Fields &f, DevScalars *s,
+                                           const PhysParams &prm, int nz, int bx,
+                                           int by, int bz)
+{
+    constexpr int NT = TX * TY;
+    constexpr int PX = TX + 1;
+    constexpr int PN = (TX + 1) * (TY + 1);
+    // node plane k's positions in slot k % 2, its velocities in slot k % 3;
+    // the forces on corners 1, 2, 3 of each thread's face of plane k in k % 2
+    __shared__ double pos[2][3][PN];
+    __shared__ double vel[3][3][PN];
+    __shared__ double side[2][3][3][NT];
+    __shared__ int s_go, s_par;
+    __shared__ double s_dt;
+
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        // the flags are only changed by earlier kernels: read them once
+        s_go = (s->active != 0 && s->error == 0) ? 1 : 0;
+        s_par = s->cur;
+        s_dt = s->deltatime;
+    }
+    __syncthreads();
+    if (!s_go) {
+        return;
+    }
+    const int par = wave_uniform(s_par);
+    const double dt = wave_uniform(s_dt);
+    const int nx = f.nx;
+    const int en = nx + 1;
+    typename Fields::CPtr in[6] = {
+        parity_copy(f.x, par ^ 1),  parity_copy(f.y, par ^ 1),  parity_copy(f.z, par ^ 1),
+        parity_copy(f.xd, par ^ 1), parity_copy(f.yd, par ^ 1), parity_copy(f.zd, par ^ 1)};
+
+    const int tx = tid % TX;
+    const int ty = tid / TX;
+    const int i0 = bx * (TX - 1);
+    const int j0 = by * (TY - 1);
+    const int kc0 = bz * nz;
+    const int kc1 = min(kc0 + nz, en);  // owned node planes [kc0, kc1)
+    // this thread's element column; the node column (ie, je) is owned when
+    // tx, ty >= 1
+    const int ie = i0 - 1 + tx;
+    const int je = j0 - 1 + ty;
+    const bool col_valid = ie >= 0 && ie < nx && je >= 0 && je < nx;
+    const bool owner = tx >= 1 && ty >= 1 && ie <= nx && je <= nx;
+    const double hgc = prm.hgcoef > 0.0 ? -prm.hgcoef * 0.01 : 0.0;
+
+    // A node plane of the tile is (TX+1) x (TY+1) nodes; thread tid holds the
+    // slots tid + r * NT (r < kSlots) of it, fetched into registers one layer
+    // ahead so that the loads overlap the element arithmetic.  Slots outside
+    // the domain hold its nearest node: the columns that read them add no
+    // force.
+    constexpr int kSlots = (PN + NT - 1) / NT;
+    unsigned gnode[kSlots];  // node index of each slot in plane 0
+#pragma unroll
+    for (int r = 0; r < kSlots; ++r) {
+        const int idx = min(tid + r * NT, PN - 1);
+        const int gi = min(max(i0 - 1 + idx % PX, 0), nx);
+        const int gj = min(max(j0 - 1 + idx / PX, 0), nx);
+        gnode[r] = unsigned(gj * en + gi);
+    }
+    const unsigned plane_stride = unsigned(en * en);
+    double pre[kSlots][6];
+    auto fetch_plane = [&](int kp) {
+#pragma unroll
+        for (int r = 0; r < kSlots; ++r) {
+            if ((r + 1) * NT <= PN || tid + r * NT < PN) {
+                const unsigned n = unsigned(kp) * plane_stride + gnode[r];
+#pragma unroll
+                for (int fld = 0; fld < 6; ++fld) {
+                    pre[r][fld] = load_at(in[fld], n);
+                }
+            }
+        }
+    };
+    auto store_plane = [&](int kp, int vslot) {
+#pragma unroll
+        for (int r = 0; r < kSlots; ++r) {
+            const int idx = tid + r * NT;
+            if ((r + 1) * NT <= PN || idx < PN) {
+#pragma unroll
+                for (int t = 0; t < 3; ++t) {
+                    pos[kp & 1][t][idx] = pre[r][t];
+                    vel[vslot][t][idx] = pre[r][3 + t];
+                }
+            }
+        }
+    };
+    const int base = ty * PX + tx;
+    auto read_face = [&](const double *p) {
+        return face_modes(p[base], p[base + 1], p[base + PX + 1], p[base + PX]);
+    };
+
+    // element fields (p, q, v, volo, ss, elemMass) of the next layer and the
+    // owned node's mass of the next plane, loaded one layer ahead; a column
+    // outside the domain keeps these values, whose forces are zero
+    double epre[6] = {0.0, 0.0, 1.0, 1.0, 0.0, 0.0};
+    double mpre = 1.0;
+    auto fetch_elem = [&](int kk) {
+        if (kk < nx && col_valid) {
+            const unsigned e = unsigned((kk * nx + je) * nx + ie);
+            epre[0] = load_at(f.p, e);
+            epre[1] = load_at(f.q, e);
+            epre[2] = load_at(f.v, e);
+            epre[3] = load_at(f.volo, e);
+            epre[4] = load_at(f.ss, e);
+            epre[5] = load_at(f.elem_mass, e);
+        }
+    };
+    auto fetch_mass = [&](int kk) {
+        if (owner && kk >= kc0 && kk < kc1) {
+            mpre = load_at(f.nodal_mass, unsigned((kk * en + je) * en + ie));
+        }
+    };
+
+    const int kbeg = (kc0 > 0) ? kc0 - 1 : 0;
+    FaceModes<double> lo[3];  // the positions' face modes of node plane k
+    double top[3][4];         // forces on the face of plane k from the layer below
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            top[t][c] = 0.0;
+        }
+    }
+    // the nodes of plane k from the forces on its face: corner 0 stays,
+    // corners 1, 2, 3 go to the threads whose node they are (:1613-1683)
+    auto stage_face = [&](int k, const double (&face)[3][4], double (&F)[3]) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const double ap = face[t][0] + face[t][1], am = face[t][0] - face[t][1];
+            const double bp = face[t][2] + face[t][3], bm = face[t][2] - face[t][3];
+            F[t] = am - bm;
+            side[k & 1][t][0][tid] = ap - bp;
+            side[k & 1][t][1][tid] = ap + bp;
+            side[k & 1][t][2][tid] = am + bm;
+        }
+    };
+    auto move_node = [&](int k, double (&F)[3], const double (&own)[6], double mass) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const double(&sd)[3][NT] = side[k & 1][t];
+            F[t] += (sd[1][tid - TX - 1] + sd[2][tid - TX]) + sd[0][tid - 1];
+        }
+        const unsigned n = unsigned((k * en + je) * en + ie);
+        const double minv = elem_recip(mass);
+        double xdd = F[0] * minv;
+        double ydd = F[1] * minv;
+        double zdd = F[2] * minv;
+        if (ie == 0) xdd = 0.0;
+        if (je == 0) ydd = 0.0;
+        if (k == 0) zdd = 0.0;
+        double xd = own[3] + xdd * dt;
+        if (fabs(xd) < prm.u_cut) xd = 0.0;
+        double yd = own[4] + ydd * dt;
+        if (fabs(yd) < prm.u_cut) yd = 0.0;
+        double zd = own[5] + zdd * dt;
+        if (fabs(zd) < prm.u_cut) zd = 0.0;
+        store_at(parity_copy(f.xd, par), n, xd);
+        store_at(parity_copy(f.yd, par), n, yd);
+        store_at(parity_copy(f.zd, par), n, zd);
+        store_at(parity_copy(f.x, par), n, own[0] + xd * dt);
+        store_at(parity_copy(f.y, par), n, own[1] + yd * dt);
+        store_at(parity_copy(f.z, par), n, own[2] + zd * dt);
+    };
+    const int klast = min(kc1, nx);  // element layers [kbeg, klast)
+    fetch_elem(kbeg);
+    fetch_mass(kbeg);
+    int v0 = 0;  // the velocity slot of plane k
+    fetch_plane(kbeg);
+    store_plane(kbeg, 0);
+    fetch_plane(kbeg + 1);  // kbeg < nx: the layer below the block's first plane exists
+    store_plane(kbeg + 1, 1);
+    if (kbeg + 1 < klast) {
+        fetch_plane(kbeg + 2);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+        lo[t] = read_face(pos[kbeg & 1][t]);
+    }
+    // Iteration k: the element layer between planes k and k + 1 (both in
+    // LDS, plane k + 2 on its way), then the nodes of plane k.  Its one
+    // barrier comes when the thread's share of plane k + 2 and of the face
+    // forces is staged; what it waits for is read before the next one, from
+    // slots that are written after that.
+    for (int k = kbeg; k < klast; ++k) {
+        const int v1 = v0 == 2 ? 0 : v0 + 1;
+        const int v2 = v1 == 2 ? 0 : v1 + 1;
+        const double mass = mpre;
+        const double press64 = (epre[0] + epre[1]) * 0.015625;
+        const double vol = epre[2];
+        const double determ = epre[3] * vol;
+        const double hgm = hgc * epre[4] * epre[5];
+        fetch_elem(k + 1);
+        fetch_mass(k + 1);
+        double own[6];
+        ForceShape<double> sh;
+        {
+            ElemModes<double> xyz[3];
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                const FaceModes<double> hi = read_face(pos[(k + 1) & 1][t]);
+                xyz[t] = elem_modes(lo[t], hi);
+                own[t] = lo[t].v0;
+                lo[t] = hi;
+            }
+            force_shape(xyz[0], xyz[1], xyz[2], elem_recip(determ), sh);
+        }
+        // VolumeError on the Jacobian volume, then on v, which the
+        // reference tests for every element before it looks at hgcoef
+        // (:1579-1584, :1540-1543)
+        if (col_valid && (sh.det <= 0.0 || vol <= 0.0)) {
+            atomicCAS(&s->error, 0, -1);
+        }
+        const double coef = hg_over_root(hgm, hg_root(determ));
+        double face[3][4];  // forces on the face of plane k, both layers
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const FaceModes<double> vlo = read_face(vel[v0][t]);
+            const ElemModes<double> u = elem_modes(vlo, read_face(vel[v1][t]));
+            own[3 + t] = vlo.v0;
+            const double n1 = t == 0 ? sh.n[0].x : t == 1 ? sh.n[0].y : sh.n[0].z;
+            const double n2 = t == 0 ? sh.n[1].x : t == 1 ? sh.n[1].y : sh.n[1].z;
+            const double n3 = t == 0 ? sh.n[2].x : t == 1 ? sh.n[2].y : sh.n[2].z;
+            const ElemModes<double> F = force_modes(sh, n1, n2, n3, press64, coef, u);
+            face[t][0] = top[t][0] - F.a3;
+            face[t][1] = top[t][1] + (F.a1 - F.h2);
+            face[t][2] = top[t][2] + (F.a2 - F.h1);
+            face[t][3] = top[t][3] + (F.h3 - F.h4);
+            top[t][0] = F.a3;
+            top[t][1] = F.a1 + F.h2;
+            top[t][2] = F.a2 + F.h1;
+            top[t][3] = F.h3 + F.h4;
+        }
+        double F[3];
+        stage_face(k, face, F);  // of no use below the block's first plane
+        if (k + 1 < klast) {
+            store_plane(k + 2, v2);
+            if (k + 2 < klast) {
+                fetch_plane(k + 3);
+            }
+        }
+        __syncthreads();
+        if (owner && k >= kc0) {
+            move_node(k, F, own, mass);
+        }
+        v0 = v1;
+    }
+    if (kc1 == en) {  // the domain's top plane: no layer above it
+        double F[3], own[6];
+        stage_face(nx, top, F);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            own[t] = lo[t].v0;
+            own[3 + t] = vel[v0][t][base];
+        }
+        __syncthreads();
+        if (owner) {
+            move_node(nx, F, own, mpre);
+        }
+    }
+}
+#else
 // One block's share of the sweep: node columns [bx*(TX-1), (bx+1)*(TX-1)) x
 // [by*(TY-1), (by+1)*(TY-1)) and node planes [bz*nz, (bz+1)*nz) of one
 // domain.
@@ -445,13 +733,25 @@ __device__ __forceinline__ void sweep_tile(const Fields &f, DevScalars *s,
         }
     }
 }
+#endif  // LULESH_FUSED
 
+// The tiles in one row, x fastest, each XCD taking a contiguous part of it:
+// a tile's halo, and the cache lines its ragged rows share with the next
+// tile's, then come from the XCD's own L2.  At 150^3 that takes the traffic
+// from 895 to 580 MB in both builds, and the fused build from 165 to 157 us;
+// the exact build, bounded by FP64 issue, stays at 290.
 template <int TX, int TY, int W>
 __global__ __launch_bounds__(TX *TY, W) void k_force_sweep(DevFields f, DevScalars *s,
                                                         PhysParams prm, int nz)
 {
-    sweep_tile<TX, TY>(f, s, prm, nz, int(blockIdx.x), int(blockIdx.y),
-                             int(blockIdx.z));
+    const int nbx = (f.nx + TX - 1) / (TX - 1), nby = (f.nx + TY - 1) / (TY - 1);
+    const int tiles = nbx * nby * ((f.nx + nz) / nz);
+    const int t = xcd_order(int(blockIdx.x), tiles);
+    if (t >= tiles) {
+        return;
+    }
+    const int r = t / nbx, bz = r / nby;
+    sweep_tile<TX, TY>(f, s, prm, nz, t - r * nbx, r - bz * nby, bz);
 }
 
 // The ensemble form: a grid walks the tile list of all members (one block
@@ -476,10 +776,9 @@ template <int TX, int TY, int W>
 hipError_t launch_shape(int nz, const DevFields &f, DevScalars *s,
                         const PhysParams &prm, hipStream_t stream)
 {
-    const int en = f.nx + 1;
-    const dim3 grid((en + TX - 2) / (TX - 1), (en + TY - 2) / (TY - 1),
-                    (en + nz - 1) / nz);
-    hipLaunchKernelGGL((k_force_sweep<TX, TY, W>), grid, dim3(TX * TY), 0, stream, f,
+    const int64_t tiles = int64_t((f.nx + TX - 1) / (TX - 1)) *
+                          ((f.nx + TY - 1) / (TY - 1)) * ((f.nx + nz) / nz);
+    hipLaunchKernelGGL((k_force_sweep<TX, TY, W>), dim3(unsigned((tiles + 7) / 8 * 8)), dim3(TX * TY), 0, stream, f,
                        s, prm, nz);
     return hipGetLastError();
 }

@@ -286,6 +286,36 @@ parity_copy(LULESH_AS_GLOBAL double *const (&t)[2], int par)
     return par != 0 ? t[1] : t[0];
 }
 
+// The work item of block b of a launch of count items, rounded up to whole
+// rounds over the 8 XCDs: blocks go to the XCDs round-robin, and each XCD
+// takes one contiguous part of the items, so that neighbouring items share
+// its L2.  A result >= count is no item.
+__device__ __forceinline__ int xcd_order(int b, int count)
+{
+    return (b & 7) * ((count + 7) >> 3) + (b >> 3);
+}
+
+// Value idx of an array, its byte offset a 32-bit number beside a scalar
+// base address (idx < 2^29; no domain has more nodes): one address
+// instruction for all the fields of an index, where a signed index costs a
+// 64-bit sum for each.
+__device__ __forceinline__ double load_at(const double *p, unsigned idx)
+{
+    return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(p) + idx * 8u);
+}
+__device__ __forceinline__ double load_at(const LULESH_AS_GLOBAL double *p, unsigned idx)
+{
+    return *(const LULESH_AS_GLOBAL double *)((const LULESH_AS_GLOBAL char *)p + idx * 8u);
+}
+__device__ __forceinline__ void store_at(double *p, unsigned idx, double v)
+{
+    *reinterpret_cast<double *>(reinterpret_cast<char *>(p) + idx * 8u) = v;
+}
+__device__ __forceinline__ void store_at(LULESH_AS_GLOBAL double *p, unsigned idx, double v)
+{
+    *(LULESH_AS_GLOBAL double *)((LULESH_AS_GLOBAL char *)p + idx * 8u) = v;
+}
+
 // Whether an ensemble member takes part in the cycle: active and without
 // error.  Both flags are read before either is tested (a short-circuit test
 // waits for the first load before it issues the second).
