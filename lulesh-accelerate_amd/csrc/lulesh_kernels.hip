@@ -741,65 +741,44 @@ __global__ __launch_bounds__(256) void k_q_eos_dt(DevFields f, DevScalars *s,
 
 namespace {
 
-// Per block: the EOS inputs of each thread's element, the inclusive prefix of
-// the evaluations beyond each element's first, and each wave's total.
+// Per block: the EOS inputs of the elements with more than one evaluation,
+// by place, and each wave's counts (ExtraDeal).
 struct RepLds {
     double in[7][256];
-    int end[256];
-    int wave_total[4];
+    int cnt[4];
 };
 
-// The EOS evaluations of a block's 256 elements beyond each one's first.  The
+// The EOS evaluations of a block's elements beyond each one's first.  The
 // thread that owns an element evaluates it once (its result is the
-// element's); the other rep - 1 evaluations of every element are dealt out
-// over all 256 threads, so a block of elements with 1, 2 and 20 repetitions
-// takes ceil(sum(rep - 1) / 256) extra passes instead of running every
-// thread 20 times.  An element's evaluations all read the same inputs and
-// give the same results: each is computed in full (its inputs pass through
-// an empty asm statement) and its result marked as used, as the reference
-// repeats the evaluation (lulesh-2.0.3/lulesh.cc:2413-2424).  Every thread
-// of the block (256, four waves) calls it.
+// element's); the others are dealt out over all 256 threads, so a block of
+// elements with 1, 2 and 20 repetitions takes ceil(sum(rep - 1) / 256) extra
+// passes instead of running every thread 20 times.  An element's evaluations
+// all read the same inputs and give the same results: each is computed in
+// full (its inputs pass through an empty asm statement) and its result
+// marked as used, as the reference repeats the evaluation
+// (lulesh-2.0.3/lulesh.cc:2413-2424).  Every thread of the block (256, four
+// waves) calls it.
 template <bool Unit>
 __device__ __forceinline__ void eos_extra_evaluations(const EosIn &a, int extra,
+                                                      const int (&classes)[2],
                                                       const EosConst &ec, RepLds &L)
 {
-    const int t = int(threadIdx.x), lane = t & 63, wave = t >> 6;
-    int incl = extra;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int o = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += o;
-    }
-    if (lane == 63) L.wave_total[wave] = incl;
-    __syncthreads();
-    int base = 0, total = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        const int v = L.wave_total[w];
-        if (w < wave) base += v;
-        total += v;
-    }
-    if (total == 0) {  // the same for every thread of the block
+    const ExtraDeal deal(extra, classes, L.cnt);
+    if (deal.total == 0) {  // the same for every thread of the block
         return;
     }
-    L.end[t] = incl + base;
-    L.in[0][t] = a.vnewc;
-    L.in[1][t] = a.e_old;
-    L.in[2][t] = a.delvc;
-    L.in[3][t] = a.p_old;
-    L.in[4][t] = a.q_old;
-    L.in[5][t] = a.qquad;
-    L.in[6][t] = a.qlin;
+    if (deal.place >= 0) {
+        L.in[0][deal.place] = a.vnewc;
+        L.in[1][deal.place] = a.e_old;
+        L.in[2][deal.place] = a.delvc;
+        L.in[3][deal.place] = a.p_old;
+        L.in[4][deal.place] = a.q_old;
+        L.in[5][deal.place] = a.qquad;
+        L.in[6][deal.place] = a.qlin;
+    }
     __syncthreads();
-    for (int w = t; w < total; w += 256) {
-        // the thread whose evaluations [end - extra, end) hold number w: the
-        // count of threads whose range ends at or before w (end is
-        // non-decreasing and end[255] = total > w, so src <= 255)
-        int src = 0;
-#pragma unroll
-        for (int step = 128; step >= 1; step >>= 1) {
-            if (L.end[src + step - 1] <= w) src += step;
-        }
+    for (int w = int(threadIdx.x); w < deal.total; w += 256) {
+        const int src = deal.owner(w);
         double b0 = L.in[0][src], b1 = L.in[1][src], b2 = L.in[2][src], b3 = L.in[3][src];
         double b4 = L.in[4][src], b5 = L.in[5][src], b6 = L.in[6][src];
         asm volatile("" : "+v"(b0), "+v"(b1), "+v"(b2), "+v"(b3), "+v"(b4), "+v"(b5),
@@ -841,10 +820,10 @@ __device__ __forceinline__ void q_eos_dt_nat_block(const F &f, DevScalars *s,
     __builtin_amdgcn_s_setprio(0);  // the evaluations yield to waves still loading
     if (ec.unit_rho0) {
         o = eos_repeat<true>(a, 1, ec);
-        eos_extra_evaluations<true>(a, extra, ec, L);
+        eos_extra_evaluations<true>(a, extra, f.eos_extra, ec, L);
     } else {
         o = eos_repeat<false>(a, 1, ec);
-        eos_extra_evaluations<false>(a, extra, ec, L);
+        eos_extra_evaluations<false>(a, extra, f.eos_extra, ec, L);
     }
     __builtin_amdgcn_s_setprio(1);  // stores and the block's reduction
     if (valid) {

@@ -115,6 +115,9 @@ struct DevFields {
     using CPtr = const double *;  // a read-only field (see DevFieldsG)
     int nx;
     int num_elem, num_node;
+    // the EOS evaluations beyond an element's first, in its light and in its
+    // costly regions: the two values that repetitions - 1 takes besides 0
+    int eos_extra[2];
     FastDiv div_nx;
     // node-centred: positions and velocities in two copies (see above)
     double *x[2], *y[2], *z[2], *xd[2], *yd[2], *zd[2];
@@ -144,6 +147,7 @@ struct DevFieldsG {
     using CPtr = const LULESH_AS_GLOBAL double *;
     int nx;
     int num_elem, num_node;
+    int eos_extra[2];  // see DevFields
     FastDiv div_nx;
     LULESH_AS_GLOBAL double *x[2], *y[2], *z[2], *xd[2], *yd[2], *zd[2];
     LULESH_AS_GLOBAL double *nodal_mass;
@@ -164,6 +168,8 @@ __device__ __forceinline__ DevFieldsG global_view(const DevFields &f)
     g.nx = f.nx;
     g.num_elem = f.num_elem;
     g.num_node = f.num_node;
+    g.eos_extra[0] = f.eos_extra[0];
+    g.eos_extra[1] = f.eos_extra[1];
     g.div_nx = f.div_nx;
     for (int c = 0; c < 2; ++c) {
         g.x[c] = (LULESH_AS_GLOBAL double *)f.x[c];
@@ -316,6 +322,64 @@ __device__ __forceinline__ void store_at(LULESH_AS_GLOBAL double *p, unsigned id
     *(LULESH_AS_GLOBAL double *)((LULESH_AS_GLOBAL char *)p + idx * 8u) = v;
 }
 
+// A block's EOS evaluations beyond each element's first, dealt out over its
+// 256 threads (four waves).  Repetitions take at most three values (LULESH
+// 2.0's regions: 1, 1 + cost, 10 (1 + cost)), so an element's extra
+// evaluations are 0, `light` or `heavy`.  The elements that have any take
+// consecutive places, the heavy ones first (place: one ballot per class),
+// and the block's evaluations are numbered round by round over the places,
+// the light elements' after the heavy ones': number w is of place w mod
+// n_heavy below n_heavy * heavy, and so on.  A binary search for the owner of
+// each evaluation, in a prefix sum of the elements' counts, cost eight
+// dependent LDS reads per pass, a quarter of the pass of a resting element.
+struct ExtraDeal {
+    int n_heavy, n_light, heavy, total_heavy, total;
+    float inv_heavy, inv_light;
+    int place;  // this thread's, -1: its element has none
+
+    // every thread of the block calls it; cnt: 4 ints of LDS, free to write
+    __device__ __forceinline__ ExtraDeal(int extra, const int (&classes)[2], int *cnt)
+    {
+        const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
+        heavy = classes[1];
+        const bool is_heavy = extra > 0 && extra == heavy;
+        const bool is_light = extra > 0 && !is_heavy;
+        const unsigned long long mh = __ballot(is_heavy), ml = __ballot(is_light);
+        if (lane == 0) {
+            cnt[wave] = __popcll(mh) | __popcll(ml) << 16;
+        }
+        __syncthreads();
+        int before = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const int c = wave_uniform(cnt[w]);
+            before += w < wave ? c : 0;
+            all += c;
+        }
+        n_heavy = all & 0xffff;
+        n_light = all >> 16;
+        total_heavy = n_heavy * heavy;
+        total = total_heavy + n_light * classes[0];
+        inv_heavy = 1.0f / float(max(n_heavy, 1));
+        inv_light = 1.0f / float(max(n_light, 1));
+        const unsigned long long below = (1ull << lane) - 1;
+        place = is_heavy   ? (before & 0xffff) + __popcll(mh & below)
+                : is_light ? n_heavy + (before >> 16) + __popcll(ml & below)
+                           : -1;
+    }
+
+    // the place of evaluation w < total; w < 2^24, so float holds it and the
+    // quotient is at most one off
+    __device__ __forceinline__ int owner(int w) const
+    {
+        const bool h = w < total_heavy;
+        const int n = h ? n_heavy : n_light;
+        const int v = h ? w : w - total_heavy;
+        const int r = v - int(float(v) * (h ? inv_heavy : inv_light)) * n;
+        return (h ? 0 : n_heavy) + (r < 0 ? r + n : r >= n ? r - n : r);
+    }
+};
+
 // Whether an ensemble member takes part in the cycle: active and without
 // error.  Both flags are read before either is tested (a short-circuit test
 // waits for the first load before it issues the second).
@@ -334,6 +398,7 @@ __device__ __forceinline__ bool member_running(const DevScalars *s)
 struct DevFieldsMixed {
     int nx;
     int num_elem, num_node;
+    int eos_extra[2];  // see DevFields
     FastDiv div_nx;
     double *x[2], *y[2], *z[2], *xd[2], *yd[2], *zd[2];
     double *nodal_mass;

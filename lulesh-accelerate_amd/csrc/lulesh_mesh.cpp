@@ -273,6 +273,19 @@ HostMesh build_mesh(const MeshConfig &cfg)
             region_rep(cfg.ic_mode, m.num_reg, cfg.cost, r));
         m.elem_rep[i] = m.eos_rep[static_cast<size_t>(slot)];
     }
+    for (int r = 0; r < m.num_reg; ++r) {
+        const int extra = region_rep(cfg.ic_mode, m.num_reg, cfg.cost, r) - 1;
+        if (extra > 0 && extra != m.eos_extra[0] && extra != m.eos_extra[1]) {
+            if (m.eos_extra[0] != 0) {
+                throw std::logic_error("build_mesh: more than three repetition counts");
+            }
+            m.eos_extra[0] = m.eos_extra[1];
+            m.eos_extra[1] = extra;
+        }
+    }
+    if (m.eos_extra[0] > m.eos_extra[1]) {
+        std::swap(m.eos_extra[0], m.eos_extra[1]);
+    }
     m.eos_blocks = eos_block_order(m.elem_rep);
     return m;
 }

@@ -39,6 +39,7 @@ struct HostMesh {
     std::vector<uint16_t> eos_rep;      // EOS repetitions at each eos_order slot
     std::vector<int32_t> region_offset; // start of each region in eos_order
     std::vector<uint16_t> elem_rep;     // EOS repetitions of each element
+    int eos_extra[2] = {0, 0};          // the values of elem_rep - 1 besides 0: light, heavy
     std::vector<int32_t> eos_blocks;    // dispatch order of the mesh-order Q/EOS blocks
 };
 

@@ -877,61 +877,41 @@ __device__ __forceinline__ void fold_minima_mixed(DevScalars *s, unsigned long l
     }
 }
 
-// Per block: the EOS inputs of each thread's element, the inclusive prefix of
-// the evaluations beyond each element's first, and each wave's total.
+// Per block: the EOS inputs of the elements with more than one evaluation,
+// by place, and each wave's counts (ExtraDeal).
 struct RepLdsMixed {
     double in_d[2][256];
     float in_f[5][256];
-    int end[256];
-    int wave_total[4];
+    int cnt[4];
 };
 
-// The EOS evaluations of a block's 256 elements beyond each one's first,
-// dealt out over all 256 threads (the scheme of eos_extra_evaluations in
+// The EOS evaluations of a block's elements beyond each one's first, dealt
+// out over all 256 threads (the scheme of eos_extra_evaluations in
 // lulesh_kernels.hip): the thread that owns an element evaluates it once and
-// keeps that result; the other rep - 1 evaluations of every element take
-// ceil(sum(rep - 1) / 256) passes of the block.  Each is computed in full
-// and its result marked as used.  Every thread of the block calls it.
+// keeps that result; the others take ceil(sum(rep - 1) / 256) passes of the
+// block.  Each is computed in full and its result marked as used.  Every
+// thread of the block calls it.
 __device__ __forceinline__ void eos_extra_evaluations_mixed(const EosInMixed &a, int extra,
+                                                            const int (&classes)[2],
                                                             const EosConstMixed &ec,
                                                             RepLdsMixed &L)
 {
-    const int t = int(threadIdx.x), lane = t & 63, wave = t >> 6;
-    int incl = extra;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int o = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += o;
-    }
-    if (lane == 63) L.wave_total[wave] = incl;
-    __syncthreads();
-    int base = 0, total = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        const int v = L.wave_total[w];
-        if (w < wave) base += v;
-        total += v;
-    }
-    if (total == 0) {  // the same for every thread of the block
+    const ExtraDeal deal(extra, classes, L.cnt);
+    if (deal.total == 0) {  // the same for every thread of the block
         return;
     }
-    L.end[t] = incl + base;
-    L.in_d[0][t] = a.vnewc;
-    L.in_d[1][t] = a.e_old;
-    L.in_f[0][t] = a.delvc;
-    L.in_f[1][t] = a.p_old;
-    L.in_f[2][t] = a.q_old;
-    L.in_f[3][t] = a.qquad;
-    L.in_f[4][t] = a.qlin;
+    if (deal.place >= 0) {
+        L.in_d[0][deal.place] = a.vnewc;
+        L.in_d[1][deal.place] = a.e_old;
+        L.in_f[0][deal.place] = a.delvc;
+        L.in_f[1][deal.place] = a.p_old;
+        L.in_f[2][deal.place] = a.q_old;
+        L.in_f[3][deal.place] = a.qquad;
+        L.in_f[4][deal.place] = a.qlin;
+    }
     __syncthreads();
-    for (int w = t; w < total; w += 256) {
-        // the thread whose evaluations [end - extra, end) hold number w
-        // (end is non-decreasing and end[255] = total > w, so src <= 255)
-        int src = 0;
-#pragma unroll
-        for (int step = 128; step >= 1; step >>= 1) {
-            if (L.end[src + step - 1] <= w) src += step;
-        }
+    for (int w = int(threadIdx.x); w < deal.total; w += 256) {
+        const int src = deal.owner(w);
         double b0 = L.in_d[0][src], b1 = L.in_d[1][src];
         float b2 = L.in_f[0][src], b3 = L.in_f[1][src], b4 = L.in_f[2][src];
         float b5 = L.in_f[3][src], b6 = L.in_f[4][src];
@@ -1007,7 +987,7 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_mixed_nat(DevFieldsMixed f, De
     }
     __builtin_amdgcn_s_setprio(0);  // the evaluations yield to waves still loading
     const EosOutMixed o = eos_repeat_mixed(a, 1, ec);
-    eos_extra_evaluations_mixed(a, extra, ec, rep_lds);
+    eos_extra_evaluations_mixed(a, extra, f.eos_extra, ec, rep_lds);
     __builtin_amdgcn_s_setprio(1);  // stores and the block's reduction
     if (valid) {
         eos_finish_mixed(f, prm, el, kp, a.vnewc, o, cand_c, cand_h);

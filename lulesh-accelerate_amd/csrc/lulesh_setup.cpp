@@ -69,6 +69,8 @@ void carve_domain(char *base, const HostMesh &m, DevFields &f, DevScalars **s)
     f.num_elem = int(m.num_elem);
     f.num_node = int(m.num_node);
     f.div_nx = make_fastdiv(unsigned(m.nx));
+    f.eos_extra[0] = m.eos_extra[0];
+    f.eos_extra[1] = m.eos_extra[1];
     for (int c = 0; c < 2; ++c) {
         f.x[c] = take_node(); f.y[c] = take_node(); f.z[c] = take_node();
         f.xd[c] = take_node(); f.yd[c] = take_node(); f.zd[c] = take_node();
@@ -169,6 +171,8 @@ void carve_domain_mixed(char *base, const HostMesh &m, DevFieldsMixed &f, DevSca
     f.num_elem = int(m.num_elem);
     f.num_node = int(m.num_node);
     f.div_nx = make_fastdiv(unsigned(m.nx));
+    f.eos_extra[0] = m.eos_extra[0];
+    f.eos_extra[1] = m.eos_extra[1];
     for (int c = 0; c < 2; ++c) {
         f.x[c] = take_node(); f.y[c] = take_node(); f.z[c] = take_node();
         f.xd[c] = take_node(); f.yd[c] = take_node(); f.zd[c] = take_node();
