@@ -67,8 +67,9 @@ def build_library() -> str:
         lang = ["-x", "hip"] if src.endswith(".hip") else []
         jobs.append((obj, [cc] + COMMON_FLAGS + ["-fPIC"] + lang +
                      ["-c", os.path.join(CSRC, src), "-o", obj]))
-    fused_flags = [("-ffp-contract=fast" if f == "-ffp-contract=off" else f)
-                   for f in COMMON_FLAGS] + ["-DLULESH_FUSED"]
+    # the sources' own pragmas say where the fused build may contract: with
+    # -ffp-contract=fast the compiler would do so everywhere
+    fused_flags = COMMON_FLAGS + ["-DLULESH_FUSED"]
     for src in FUSED_SOURCES:
         obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + "_fused.o")
         jobs.append((obj, [cc] + fused_flags + ["-fPIC", "-x", "hip", "-c",

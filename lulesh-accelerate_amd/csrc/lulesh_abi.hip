@@ -85,6 +85,49 @@ int default_sweep_planes(int nx)
     return 1;
 }
 
+// Planes (or layers) per block of a sweep that cuts `planes` of them into
+// chunks, `cols` blocks each, `resident` of which a CU holds.  A block takes
+// its planes one after another, so a launch lasts as many rounds of the
+// resident slots as it has, times a block's planes and the `extra` it costs
+// to start (the recomputed halo planes, and about two more for the first
+// loads).  The fewest plane times win, the longer chunk of two equals: its
+// halo is a smaller part.  For the kinematics sweep it picks the
+// fastest of a scan at 150^3 (10 layers, 1.95 rounds, 133 us; 9: 157 us) and
+// 180^3 (12, 2.8 rounds, 225 us; 30: 286 us).
+int plan_planes(int planes, long long cols, int resident, int extra, int most)
+{
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
+            hipSuccess ||
+        cus < 1) {
+        cus = 256;
+    }
+    const long long slots = (long long)resident * cus;
+    int best = 1;
+    long long best_cost = -1;
+    for (int nz = 1; nz <= std::min(planes, most); ++nz) {
+        const long long blocks = cols * ((planes + nz - 1) / nz);
+        const long long cost = (blocks + slots - 1) / slots * (nz + extra);
+        if (best_cost < 0 || cost <= best_cost) {
+            best_cost = cost;
+            best = nz;
+        }
+    }
+    return best;
+}
+
+// Whether the fused step's kinematics and limiter run as one sweep.  The
+// sweep saves half the memory traffic of the two kernels apart and costs a
+// sixth more arithmetic and two barriers a layer, so it pays once a domain's
+// fields no longer fit in the 256 MB last-level cache: kinematics plus Q/EOS
+// 210 against 253 us at 150^3, 92 against 99 us at 110^3, but 66 against
+// 57 us at 91^3.
+bool limiter_in_sweep(int64_t num_elem, int64_t num_node)
+{
+    return (19 * num_elem + 13 * num_node) * 8 > (int64_t(256) << 20);
+}
+
 struct TimedLaunch {
     int kernel;
     hipEvent_t start, stop;
@@ -121,6 +164,8 @@ struct lulesh_domain {
     DevScalars *s = nullptr;
     PhysParams prm{};
     SweepShape sweep = kDefaultSweep;
+    bool limit_sweep = false;  // the fused kinematics and limiter in one sweep
+    int limit_planes = 1;      //   and its element layers per block
     void *arena = nullptr;
     hipStream_t stream = nullptr;
 
@@ -253,7 +298,9 @@ int queue_cycle_u(lulesh_domain *d)
     return LULESH_OK;
 }
 
-int queue_cycle(lulesh_domain *d)
+// store: whether the fused cycle leaves the intermediate fields (delv, the Q
+// gradients) in memory: the last cycle of a call does
+int queue_cycle(lulesh_domain *d, bool store)
 {
     if (d->unstructured) {
         return queue_cycle_u(d);
@@ -279,6 +326,17 @@ int queue_cycle(lulesh_domain *d)
                           : launch_force_sweep(d->sweep, f, s, p, st);
          })))
         return rc;
+    // unless another Q phase is set (the learned closure, the region-sorted
+    // schedule)
+    if (fused && d->limit_sweep && !d->learned && d->eos_bands == 0) {
+        if ((rc = launch(d, KID_KINEMATICS_Q, [&]() -> hipError_t {
+                 return fused::launch_kinematics_limit(f, s, p, d->limit_planes, store, st);
+             })))
+            return rc;
+        return launch(d, KID_Q_EOS_DT, [&] {
+            hipLaunchKernelGGL(fused::k_eos_dt_nat, dim3(ge), dim3(kBlock), 0, st, f, s, p);
+        });
+    }
     if ((rc = launch(d, KID_KINEMATICS_Q, [&] {
              if (mixed) {
                  hipLaunchKernelGGL(k_kinematics_q_mixed, dim3(ge), dim3(kBlock), 0, st, fm,
@@ -335,6 +393,8 @@ std::vector<unsigned char> launch_signature(const lulesh_domain *d)
     put(&d->s, sizeof(d->s));
     put(&d->prm, sizeof(d->prm));
     put(&d->sweep, sizeof(d->sweep));
+    put(&d->limit_sweep, sizeof(d->limit_sweep));
+    put(&d->limit_planes, sizeof(d->limit_planes));
     put(&d->mesh, sizeof(d->mesh));
     put(&d->fblocks, sizeof(d->fblocks));
     return sig;
@@ -361,7 +421,7 @@ int ensure_graph(lulesh_domain *d)
     HIP_TRY(d, hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
     int rc = LULESH_OK;
     for (int c = 0; c < kGraphCycles && rc == LULESH_OK; ++c) {
-        rc = queue_cycle(d);
+        rc = queue_cycle(d, c + 1 == kGraphCycles);
     }
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(d->stream, &g);
@@ -558,7 +618,10 @@ int create_domain(const lulesh_config *cfg, bool mixed, double efactor,
     d->mixed = mixed;
     d->sweep = mixed ? kDefaultSweepMixed : kDefaultSweep;
     if (!mixed && cfg->nx >= 1 && cfg->nx <= 600) {
+        const int64_t nx = cfg->nx;
         d->sweep.nz = default_sweep_planes(cfg->nx);
+        d->limit_sweep = limiter_in_sweep(nx * nx * nx, (nx + 1) * (nx + 1) * (nx + 1));
+        d->limit_planes = plan_planes(cfg->nx, fused::kinematics_limit_columns(cfg->nx), 3, 5, 64);
     }
     HostMesh m;
     try {
@@ -933,7 +996,7 @@ int lulesh_step(lulesh_domain *d, int ncycles, int *cycles_done)
         }
     }
     for (; c < ncycles; ++c) {
-        if ((rc = queue_cycle(d))) return rc;
+        if ((rc = queue_cycle(d, c + 1 == ncycles))) return rc;
     }
     // the last cycle's time constraints (the others were applied by the
     // following cycle's TimeIncrement)

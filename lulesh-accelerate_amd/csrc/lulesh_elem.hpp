@@ -47,16 +47,16 @@ namespace lulesh {
 // 1 / b and a / b in the element arithmetic.  The bit-identical build
 // divides, correctly rounded, as the reference does.  The fused build, held
 // to the reference's tolerances rather than to its bits, multiplies by the
-// hardware reciprocal estimate refined by two Newton steps (b finite, normal
-// and nonzero): five instructions where the divide sequence takes ten.  In
+// hardware reciprocal estimate (relative error below 2^-23) with one
+// third-order step (b finite, normal and nonzero): four instructions where
+// the divide sequence takes ten.  In
 // float (the mixed-precision step) these are plain divides.
 __device__ __forceinline__ double elem_recip(double b)
 {
 #ifdef LULESH_FUSED
-    double r = __builtin_amdgcn_rcp(b);
-    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
-    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
-    return r;
+    const double r = __builtin_amdgcn_rcp(b);
+    const double e = __builtin_fma(-b, r, 1.0);
+    return __builtin_fma(r, __builtin_fma(e, e, e), r);
 #else
     return 1.0 / b;
 #endif
@@ -460,13 +460,13 @@ __device__ __forceinline__ EosOut eos_element(double vnewc, double e_old,
     }
     const double bvc_half = c1s * r_half, bvc = c1s * r;
     const double pq_old = p_old + q_old;
-    double e_new = e_old - 0.5 * delvc * pq_old;
+    double e_new = __builtin_fma(-0.5 * delvc, pq_old, e_old);
     if (e_new < c.emin) e_new = c.emin;
     const double p_half = eos_pressure(bvc_half, e_new, vnewc, c);
     const bool expanding = delvc > 0.;
     // c1s e + v^2 bvc p, the sound speed squared times rho0
     auto sound = [&](double v, double e, double p) {
-        double s = c1s * (e + v * p);
+        double s = c1s * __builtin_fma(v, p, e);
         if (!UnitRho0) {
             s = s / c.rho0;
         }
@@ -474,25 +474,26 @@ __device__ __forceinline__ EosOut eos_element(double vnewc, double e_old,
     };
     double q_new = 0.;
     if (!expanding) {
-        q_new = sound(vhalf, e_new, p_half) * ql_old + qq_old;
+        q_new = __builtin_fma(sound(vhalf, e_new, p_half), ql_old, qq_old);
     }
     const double pq_half = p_half + q_new;
-    e_new = e_new + 0.5 * delvc * (3.0 * pq_old - 4.0 * pq_half);
+    e_new = __builtin_fma(0.5 * delvc, __builtin_fma(3.0, pq_old, -4.0 * pq_half), e_new);
     if (fabs(e_new) < c.e_cut) e_new = 0.;
     if (e_new < c.emin) e_new = c.emin;
     double p_new = eos_pressure(bvc, e_new, vnewc, c);
     double q_tilde = 0.;
     if (!expanding) {
-        q_tilde = sound(v2r, e_new, p_new) * ql_old + qq_old;
+        q_tilde = __builtin_fma(sound(v2r, e_new, p_new), ql_old, qq_old);
     }
-    e_new = e_new - (7.0 * pq_old - 8.0 * pq_half + (p_new + q_tilde)) * (delvc * (1.0 / 6.0));
+    const double sum = __builtin_fma(7.0, pq_old, __builtin_fma(-8.0, pq_half, p_new + q_tilde));
+    e_new = __builtin_fma(-sum, delvc * (1.0 / 6.0), e_new);
     if (fabs(e_new) < c.e_cut) e_new = 0.;
     if (e_new < c.emin) e_new = c.emin;
     p_new = eos_pressure(bvc, e_new, vnewc, c);
     EosOut o;
     o.ss = sound(v2r, e_new, p_new);
     if (delvc <= 0.) {
-        q_new = o.ss * ql_old + qq_old;
+        q_new = __builtin_fma(o.ss, ql_old, qq_old);
         if (fabs(q_new) < c.q_cut) q_new = 0.;
     }
     o.p = p_new;

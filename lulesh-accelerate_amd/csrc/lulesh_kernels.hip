@@ -23,6 +23,9 @@
 #include "lulesh_kernels.hpp"
 
 #include "lulesh_elem.hpp"
+#ifdef LULESH_FUSED
+#include "lulesh_modal.hpp"
+#endif
 #include "lulesh_mlp.hpp"
 
 // FMA contraction off: every value rounded as the reference rounds it;
@@ -39,6 +42,20 @@ LULESH_VARIANT_BEGIN
 namespace {
 
 constexpr double kBig = 1.0e+20;
+
+// a * b + c: two roundings in the bit-identical build, one in the fused
+// build.  Where the fused build has to give the same bits from two kernels,
+// its multiply-adds are written out like this rather than left to the
+// compiler, whose choice depends on what surrounds them (and contraction is
+// off where they stand).
+__device__ __forceinline__ double madd(double a, double b, double c)
+{
+#ifdef LULESH_FUSED
+    return __builtin_fma(a, b, c);
+#else
+    return a * b + c;
+#endif
+}
 
 __device__ __forceinline__ unsigned long long as_bits(double v)
 {
@@ -76,6 +93,13 @@ __device__ __forceinline__ void apply_constraints(DevScalars *s, int ic_mode)
     }
     if (c < kBig) s->dtcourant = c;
     if (h < kBig) s->dthydro = h;
+}
+
+// a + b of two products, each rounded on its own
+__device__ __forceinline__ double add(double a, double b)
+{
+#pragma clang fp contract(off)
+    return a + b;
 }
 
 // element (i, j, k) of a flat element index
@@ -140,6 +164,7 @@ __device__ __forceinline__ void time_increment(DevScalars *s, int ic_mode)
     s->time += s->deltatime;
     ++s->cycle;
     s->cur ^= 1;  // this cycle's nodes go to the other copy
+    s->last = (!(s->time < s->stoptime) || !(s->cycle < s->max_cycles)) ? 1 : 0;
     s->acc_courant = as_bits(kBig);
     s->acc_hydro = as_bits(kBig);
     s->dt_pending = 1;
@@ -195,7 +220,8 @@ __device__ __forceinline__ void kinematics_q_nodes(const F &f, DevScalars *s,
     typename F::CPtr __restrict__ pxd = parity_copy(f.xd, par);
     typename F::CPtr __restrict__ pyd = parity_copy(f.yd, par);
     typename F::CPtr __restrict__ pzd = parity_copy(f.zd, par);
-    double x[8], y[8], z[8], xv[8], yv[8], zv[8];
+    double xyz[3][8], xv[8], yv[8], zv[8];
+    double(&x)[8] = xyz[0], (&y)[8] = xyz[1], (&z)[8] = xyz[2];
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
         x[c] = px[nodes[c]];
@@ -221,6 +247,24 @@ __device__ __forceinline__ void kinematics_q_nodes(const F &f, DevScalars *s,
         __builtin_amdgcn_s_setprio(1);  // a wave with its data finishes first
     }
 
+#ifdef LULESH_FUSED
+    const ElemModes<double> mu = corner_modes(xv), mv = corner_modes(yv), mw = corner_modes(zv);
+    const Vec3<double> u[3] = {{mu.a1, mv.a1, mw.a1}, {mu.a2, mv.a2, mw.a2}, {mu.a3, mv.a3, mw.a3}};
+    const ElemKinematics r = elem_kinematics(elem_shape(xyz), u, volo, dt);
+    f.vnew[el] = r.vnew;
+    f.delv[el] = r.vnew - v_old;
+    f.arealg[el] = r.arealg;
+    f.vdov[el] = r.vdov;
+    f.delv_xi[el] = r.delv[0];
+    f.delv_eta[el] = r.delv[1];
+    f.delv_zeta[el] = r.delv[2];
+    f.delx_xi[el] = r.delx[0];
+    f.delx_eta[el] = r.delx[1];
+    f.delx_zeta[el] = r.delx[2];
+    if (r.vnew <= 0.0) {
+        raise_error(s, -1);
+    }
+#else
     // kinematics
     const double volume = elem_volume(x, y, z);
     const double vnew = elem_quot(volume, volo);
@@ -301,6 +345,7 @@ __device__ __forceinline__ void kinematics_q_nodes(const F &f, DevScalars *s,
     dyv = -0.25 * ((yv[0] + yv[1] + yv[5] + yv[4]) - (yv[3] + yv[2] + yv[6] + yv[7]));
     dzv = -0.25 * ((zv[0] + zv[1] + zv[5] + zv[4]) - (zv[3] + zv[2] + zv[6] + zv[7]));
     f.delv_eta[el] = ax * dxv + ay * dyv + az * dzv;
+#endif  // LULESH_FUSED
 }
 
 template <class F>
@@ -378,6 +423,7 @@ __device__ __forceinline__ double mono_phi(double self, double delvm,
                                            double delvp, double limiter_mult,
                                            double max_slope)
 {
+#pragma clang fp contract(off)
     const double ptiny = 1.e-36;
     const double norm = elem_recip(self + ptiny);
     double phi;
@@ -494,6 +540,7 @@ template <class F>
 __device__ __forceinline__ void q_inputs_rest(const F &f, int el, double dvxi,
                                               double dveta, double dvzeta, QInputs &in)
 {
+#pragma clang fp contract(off)
     in.vdov = f.vdov[el];
     in.vnew = f.vnew[el];
     in.volo = f.volo[el];
@@ -521,22 +568,43 @@ __device__ __forceinline__ void q_inputs_rest(const F &f, int el, double dvxi,
     }
 }
 
-// linear and quadratic Q of the monotonic limiter (:2289-2316)
-__device__ __forceinline__ void monotonic_q(const PhysParams &prm, const QInputs &in,
+// The sums of the limiter's linear and quadratic Q over the directions
+// (:2289-2316), xi and eta first, and the Q they give.
+struct QSums {
+    double lin, quad;
+};
+
+__device__ __forceinline__ QSums q_sums_xi_eta(double dxi, double phixi, double deta,
+                                               double phieta)
+{
+#pragma clang fp contract(off)
+    // rounded alike in both directions
+    const double lx = dxi * (1. - phixi), ly = deta * (1. - phieta);
+    const double qx = dxi * dxi * madd(-phixi, phixi, 1.);
+    const double qy = deta * deta * madd(-phieta, phieta, 1.);
+    return {add(lx, ly), add(qx, qy)};
+}
+
+__device__ __forceinline__ void q_from_sums(const PhysParams &prm, const QSums &s, double dzeta,
+                                            double phizeta, double rho, bool expanding,
                                             double &qlin, double &qquad)
 {
-    if (in.vdov > 0.) {
+#pragma clang fp contract(off)
+    if (expanding) {
         qlin = 0.;
         qquad = 0.;
     } else {
-        const double dxi = in.du[0], deta = in.du[1], dzeta = in.du[2];
-        const double phixi = in.phi[0], phieta = in.phi[1], phizeta = in.phi[2];
-        qlin = -prm.qlc_monoq * in.rho *
-               (dxi * (1. - phixi) + deta * (1. - phieta) + dzeta * (1. - phizeta));
-        qquad = prm.qqc_monoq * in.rho *
-                (dxi * dxi * (1. - phixi * phixi) + deta * deta * (1. - phieta * phieta) +
-                 dzeta * dzeta * (1. - phizeta * phizeta));
+        qlin = -prm.qlc_monoq * rho * madd(dzeta, 1. - phizeta, s.lin);
+        qquad = prm.qqc_monoq * rho *
+                madd(dzeta * dzeta, madd(-phizeta, phizeta, 1.), s.quad);
     }
+}
+
+__device__ __forceinline__ void monotonic_q(const PhysParams &prm, const QInputs &in,
+                                            double &qlin, double &qquad)
+{
+    q_from_sums(prm, q_sums_xi_eta(in.du[0], in.phi[0], in.du[1], in.phi[1]), in.du[2],
+                in.phi[2], in.rho, in.vdov > 0., qlin, qquad);
 }
 
 // What one EOS evaluation of an element reads (the clamped new volume and
@@ -562,17 +630,12 @@ __device__ __forceinline__ EosConst eos_const(const PhysParams &prm)
     return ec;
 }
 
-// The element's side of the EOS before its evaluations: ql / qq stored,
-// qstop tested on the q of the previous cycle (:2368-2381), the new and old
+// The element's side of the EOS before its evaluations: qstop tested on the q of the previous cycle (:2368-2381), the new and old
 // relative volumes clamped (:2704-2753; 2.0 clamps vnew in place) and the
 // clamped old volume tested.
-template <class F>
-__device__ __forceinline__ EosIn eos_prepare(const F &f, DevScalars *s,
-                                             const PhysParams &prm, int el,
+__device__ __forceinline__ EosIn eos_prepare(DevScalars *s, const PhysParams &prm,
                                              const QInputs &in, double qlin, double qquad)
 {
-    f.ql[el] = qlin;
-    f.qq[el] = qquad;
     const double q_old = in.q_old;
     if (q_old > prm.qstop) {
         raise_error(s, -2);
@@ -637,7 +700,7 @@ __device__ __forceinline__ void eos_finish(const F &f, const PhysParams &prm, in
     double tmpv = (prm.ic_mode == 1) ? vnew : vnewc;
     if (fabs(tmpv - 1.0) < prm.v_cut) tmpv = 1.0;
     f.v[el] = tmpv;
-    if (prm.ic_mode == 2) {
+    if (prm.ic_mode == 2 && vnewc != vnew) {  // memory holds vnew already
         f.vnew[el] = vnewc;
     }
     if (vdov != 0.) {
@@ -645,7 +708,7 @@ __device__ __forceinline__ void eos_finish(const F &f, const PhysParams &prm, in
         const double qqc2 = 64.0 * prm.qqc * prm.qqc;
         double dtf = o.ss * o.ss;
         if (vdov < 0.) {
-            dtf = dtf + qqc2 * arealg * arealg * vdov * vdov;
+            dtf = madd(qqc2 * arealg * arealg * vdov, vdov, dtf);
         }
         dtf = sqrt(dtf);
         dtf = elem_quot(arealg, dtf);
@@ -665,7 +728,9 @@ __device__ __forceinline__ void eos_dt_elem(const F &f, DevScalars *s,
                                             unsigned long long &cand_c,
                                             unsigned long long &cand_h)
 {
-    const EosIn a = eos_prepare(f, s, prm, el, in, qlin, qquad);
+    f.ql[el] = qlin;
+    f.qq[el] = qquad;
+    const EosIn a = eos_prepare(s, prm, in, qlin, qquad);
     const EosConst ec = eos_const(prm);
     EosOut o;
     __builtin_amdgcn_s_setprio(0);  // the repetitions yield to waves still loading
@@ -792,31 +857,19 @@ __device__ __forceinline__ void eos_extra_evaluations(const EosIn &a, int extra,
 
 namespace {
 
-// One block of 256 elements in mesh order, el the thread's element; every
-// thread of the block calls it (the minima are reduced over the block).
+// The EOS of one block of 256 elements in mesh order, el the thread's element
+// (valid: it has one), its inputs loaded; every thread of the block calls it
+// (the minima are reduced over the block).
 template <class F>
-__device__ __forceinline__ void q_eos_dt_nat_block(const F &f, DevScalars *s,
-                                                   const PhysParams &prm, int el,
-                                                   unsigned long long *lds_c,
-                                                   unsigned long long *lds_h, RepLds &L)
+__device__ __forceinline__ void eos_nat_block(const F &f, DevScalars *s, const PhysParams &prm,
+                                              int el, bool valid, const QInputs &in,
+                                              const EosIn &a, int extra,
+                                              unsigned long long *lds_c,
+                                              unsigned long long *lds_h, RepLds &L)
 {
-    const bool valid = el < f.num_elem;
     unsigned long long cand_c = as_bits(kBig), cand_h = as_bits(kBig);
     const EosConst ec = eos_const(prm);
-    QInputs in;
-    EosIn a{1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     EosOut o;
-    int extra = 0;
-    if (valid) {
-        const int rep = f.rep[el];
-        extra = rep - 1;
-        int i, j, k;
-        elem_ijk(f, el, i, j, k);
-        q_inputs(f, prm, el, i, j, k, in);
-        double qlin, qquad;
-        monotonic_q(prm, in, qlin, qquad);
-        a = eos_prepare(f, s, prm, el, in, qlin, qquad);
-    }
     __builtin_amdgcn_s_setprio(0);  // the evaluations yield to waves still loading
     if (ec.unit_rho0) {
         o = eos_repeat<true>(a, 1, ec);
@@ -830,6 +883,32 @@ __device__ __forceinline__ void q_eos_dt_nat_block(const F &f, DevScalars *s,
         eos_finish(f, prm, el, in, a.vnewc, o, cand_c, cand_h);
     }
     fold_minima(s, cand_c, cand_h, lds_c, lds_h);
+}
+
+// The limiter and the EOS of such a block.
+template <class F>
+__device__ __forceinline__ void q_eos_dt_nat_block(const F &f, DevScalars *s,
+                                                   const PhysParams &prm, int el,
+                                                   unsigned long long *lds_c,
+                                                   unsigned long long *lds_h, RepLds &L)
+{
+    const bool valid = el < f.num_elem;
+    QInputs in;
+    EosIn a{1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int extra = 0;
+    if (valid) {
+        const int rep = f.rep[el];
+        extra = rep - 1;
+        int i, j, k;
+        elem_ijk(f, el, i, j, k);
+        q_inputs(f, prm, el, i, j, k, in);
+        double qlin, qquad;
+        monotonic_q(prm, in, qlin, qquad);
+        f.ql[el] = qlin;
+        f.qq[el] = qquad;
+        a = eos_prepare(s, prm, in, qlin, qquad);
+    }
+    eos_nat_block(f, s, prm, el, valid, in, a, extra, lds_c, lds_h, L);
 }
 
 }  // namespace
@@ -859,6 +938,334 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_nat(DevFields f, DevScalars *s
     q_eos_dt_nat_block(f, s, prm, b * int(blockDim.x) + int(threadIdx.x), lds_c, lds_h,
                        rep_lds);
 }
+
+#ifdef LULESH_FUSED
+namespace {
+
+// Kinematics and the monotonic-Q limiter of the elements, in one sweep.
+//
+// k_kinematics_q and k_q_eos_dt_nat exchange ten fields of every element
+// through memory so that the limiter sees its neighbours' velocity
+// gradients: 1298 MB for the two at 150^3, 253 us, the rate a copy reaches.
+// Here a block owns TX x TY element columns and nz layers of them and sweeps
+// upward, one thread per column.  The gradients of a layer in xi and eta
+// reach the neighbouring threads through LDS; the one in zeta waits in its
+// own thread for the layer above.  The gradients just outside the tile are
+// formed again by 2 (TX + TY) of the threads, those of the layers below and
+// above it by every thread.  Out go vnew, the rate of volume change, the
+// characteristic length and the two Q terms, which k_eos_dt_nat reads beside
+// its own state; the other seven fields only where the cycle is one whose
+// fields a caller can read (`store`, or the run ends with it).
+//
+// At 150^3: 449 MB and 133 us here, 358 MB and 83 us for the EOS.  43 M vector
+// instructions, half of the time's issue; three waves per SIMD (168 VGPRs)
+// wait for each other at the two barriers of a layer.  What did not help:
+// the next plane held in registers across a layer (two waves, 142 us, or
+// spills, 300 us), tiles of 32 x 8 (145 us) and 64 x 4 (185 us).
+template <int TX, int TY>
+__device__ __forceinline__ void kinematics_limit_tile(const DevFields &f, DevScalars *s,
+                                                      const PhysParams &prm, int nz, bool store,
+                                                      int bx, int by, int bz)
+{
+#pragma clang fp contract(off)
+    constexpr int NT = TX * TY, PX = TX + 3, PN = (TX + 3) * (TY + 3);
+    constexpr int kHalo = 2 * (TX + TY);
+    static_assert(kHalo <= NT, "one halo gradient per thread");
+    __shared__ double plane[2][6][PN];      // node planes k and k + 1, one node around the tile
+    // the gradients of a layer, one element around the tile: xi in rows of
+    // TX + 2, then eta in rows of TX
+    constexpr int kEta = TY * (TX + 2);
+    __shared__ double grad[kEta + (TY + 2) * TX];
+    // what a thread keeps of the layer below until it knows the gradient
+    // above: here and not in registers, which decide the occupancy
+    __shared__ double below[5][NT];
+    const int par = s->cur;
+    const double dt = s->deltatime;
+    const double *const in[6] = {f.x[par], f.y[par], f.z[par], f.xd[par], f.yd[par], f.zd[par]};
+    const int nx = f.nx, en = nx + 1;
+    const int tid = int(threadIdx.x), tx = tid % TX, ty = tid / TX;
+    const int i0 = bx * TX, j0 = by * TY;
+    const int k0 = bz * nz, k1 = min(k0 + nz, nx);  // owned layers [k0, k1)
+    const int i = i0 + tx, j = j0 + ty;
+    const bool own = i < nx && j < nx;
+    store = store || s->last != 0;
+
+    constexpr int kSlots = (PN + NT - 1) / NT;
+    unsigned gnode[kSlots];  // node of plane 0 in each slot, the nearest outside the domain
+#pragma unroll
+    for (int r = 0; r < kSlots; ++r) {
+        const int idx = min(tid + r * NT, PN - 1);
+        const int gi = min(max(i0 - 1 + idx % PX, 0), nx);
+        const int gj = min(max(j0 - 1 + idx / PX, 0), nx);
+        gnode[r] = unsigned(gj * en + gi);
+    }
+    double pre[kSlots][6];
+    auto fetch_plane = [&](int kp) {
+#pragma unroll
+        for (int r = 0; r < kSlots; ++r) {
+            const unsigned n = unsigned(kp * en * en) + gnode[r];
+#pragma unroll
+            for (int t = 0; t < 6; ++t) {
+                pre[r][t] = load_at(in[t], n);
+            }
+        }
+    };
+    auto store_plane = [&](int kp) {
+#pragma unroll
+        for (int r = 0; r < kSlots; ++r) {
+            if ((r + 1) * NT <= PN || tid + r * NT < PN) {
+#pragma unroll
+                for (int t = 0; t < 6; ++t) {
+                    plane[kp & 1][t][tid + r * NT] = pre[r][t];
+                }
+            }
+        }
+    };
+    // the eight corner values of field t of the element whose first corner
+    // is the plane's slot `at`
+    auto corners = [&](int k, int t, int at, double (&v)[8]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const double *p = plane[(k + h) & 1][t] + at;
+            v[4 * h] = p[0];
+            v[4 * h + 1] = p[1];
+            v[4 * h + 2] = p[PX + 1];
+            v[4 * h + 3] = p[PX];
+        }
+    };
+    auto shape = [&](int k, int at) {
+        double xyz[3][8];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            corners(k, t, at, xyz[t]);
+        }
+        return elem_shape(xyz);
+    };
+    const int at = (ty + 1) * PX + tx + 1;
+    const unsigned elem_ji = unsigned(min(j, nx - 1) * nx + min(i, nx - 1));
+    auto elem_of = [&](int k) { return unsigned(k * nx * nx) + elem_ji; };
+
+    // The gradients around the tile: number [0, 2 TY) the columns left and
+    // right of it (xi), the rest those below and above it (eta).  Every other
+    // block gives them to its last threads, so that no SIMD has all of them.
+    const int h = (blockIdx.x & 8) ? NT - 1 - tid : tid;
+    const bool eta = h >= 2 * TY;
+    const int hg = eta ? h - 2 * TY : h;
+    const int hside = hg >= (eta ? TX : TY) ? 1 : 0;
+    const int hpos = hg - hside * (eta ? TX : TY);
+    const int hx = eta ? hpos : (hside ? TX : -1), hy = eta ? (hside ? TY : -1) : hpos;
+    const bool halo = h < kHalo && i0 + hx >= 0 && i0 + hx < nx && j0 + hy >= 0 && j0 + hy < nx;
+    const int hat = (hy + 1) * PX + hx + 1;
+    const unsigned halo_ji = halo ? unsigned((j0 + hy) * nx + i0 + hx) : elem_ji;
+    const int hgrad = eta ? kEta + (hy + 1) * TX + hx : hy * (TX + 2) + hx + 1;
+    // element fields, loaded one layer ahead
+    double volo, v_old, mass, hvolo;
+    auto fetch_elem = [&](int k) {
+        volo = load_at(f.volo, elem_of(k));
+        v_old = load_at(f.v, elem_of(k));
+        mass = load_at(f.elem_mass, elem_of(k));
+        hvolo = load_at(f.volo, unsigned(k * nx * nx) + halo_ji);
+    };
+
+    const double lm = prm.monoq_limiter_mult, ms = prm.monoq_max_slope;
+    constexpr double kExpanding = -1.0;  // in place of the density, which q does not need there
+    double dz = 0.0;  // the zeta gradient of the layer below the current one
+    auto finish = [&](int k, double dz_above) {  // the Q terms of layer k
+        const double dz_below = k == 0 ? dz : below[0][tid];
+        const double phi = mono_phi(dz, dz_below, dz_above, lm, ms);
+        const double rho = below[4][tid];
+        double qlin, qquad;
+        q_from_sums(prm, QSums{below[1][tid], below[2][tid]}, below[3][tid], phi, rho,
+                    rho == kExpanding, qlin, qquad);
+        if (own) {
+            store_at(f.ql, elem_of(k), qlin);
+            store_at(f.qq, elem_of(k), qquad);
+        }
+    };
+
+    const int kb = max(k0 - 1, 0), ke = min(k1 + 1, nx);  // layers the sweep visits
+    fetch_plane(kb);
+    store_plane(kb);
+    fetch_plane(kb + 1);
+    fetch_elem(kb);
+    store_plane(kb + 1);
+    for (int k = kb; k < ke; ++k) {
+        __syncthreads();  // planes k and k + 1 are in LDS
+        // the waves with gradients around the tile go first, then those near
+        // the barrier (142 -> 133 us at 150^3)
+        __builtin_amdgcn_s_setprio(1);
+        const bool full = k >= k0 && k < k1;
+        if (full && halo) {
+            const ElemShape hs = shape(k, hat);
+            double u[3];
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                double v[8];
+                corners(k, 3 + t, hat, v);
+                const ElemModes<double> m = corner_modes(v);
+                u[t] = eta ? m.a2 : m.a1;
+            }
+            grad[hgrad] = elem_gradient(hs.volume, hs.a, Vec3<double>{u[0], u[1], u[2]}, hvolo, eta);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        const ElemShape es = shape(k, at);
+        // the positions' registers go to the velocities and the next layer's
+        // fields
+        __builtin_amdgcn_sched_barrier(0);
+        const double volo_k = volo, v_old_k = v_old, mass_k = mass;
+        fetch_elem(min(k + 1, ke - 1));
+        Vec3<double> u[3];
+        {
+            double v[8];
+            corners(k, 3, at, v);
+            const ElemModes<double> mu = corner_modes(v);
+            corners(k, 4, at, v);
+            const ElemModes<double> mv = corner_modes(v);
+            corners(k, 5, at, v);
+            const ElemModes<double> mw = corner_modes(v);
+            u[0] = {mu.a1, mv.a1, mw.a1};
+            u[1] = {mu.a2, mv.a2, mw.a2};
+            u[2] = {mu.a3, mv.a3, mw.a3};
+        }
+        const ElemKinematics r = elem_kinematics(es, u, volo_k, dt);
+        const double dz_here = r.delv[2];
+        const int gx = ty * (TX + 2) + tx + 1, gy = kEta + (ty + 1) * TX + tx;
+        grad[gx] = r.delv[0];
+        grad[gy] = r.delv[1];
+        __builtin_amdgcn_s_setprio(2);
+        __syncthreads();  // gradients staged, plane k read
+        if (k > k0) {
+            finish(k - 1, dz_here);
+        }
+        below[0][tid] = dz;
+        dz = dz_here;
+        if (full) {
+            const double xm = grad[gx - 1], xp = grad[gx + 1];
+            const double ym = grad[gy - TX], yp = grad[gy + TX];
+            const double dx = r.delv[0], dy = r.delv[1];
+            const double phix = mono_phi(dx, i == 0 ? dx : xm, i == nx - 1 ? 0.0 : xp, lm, ms);
+            const double phiy = mono_phi(dy, j == 0 ? dy : ym, j == nx - 1 ? 0.0 : yp, lm, ms);
+            double dux = dx * r.delx[0], duy = dy * r.delx[1];
+            double duz = dz * r.delx[2];
+            if (dux > 0.) dux = 0.;
+            if (duy > 0.) duy = 0.;
+            if (duz > 0.) duz = 0.;
+            const QSums sums = q_sums_xi_eta(dux, phix, duy, phiy);
+            below[1][tid] = sums.lin;
+            below[2][tid] = sums.quad;
+            below[3][tid] = duz;
+            below[4][tid] = r.vdov > 0. ? kExpanding : elem_quot(mass_k, volo_k * r.vnew);
+            if (own) {
+                const unsigned e = elem_of(k);
+                store_at(f.vnew, e, r.vnew);
+                store_at(f.vdov, e, r.vdov);
+                store_at(f.arealg, e, r.arealg);
+                if (store) {
+                    store_at(f.delv, e, r.vnew - v_old_k);
+                    store_at(f.delv_xi, e, r.delv[0]);
+                    store_at(f.delv_eta, e, r.delv[1]);
+                    store_at(f.delv_zeta, e, r.delv[2]);
+                    store_at(f.delx_xi, e, r.delx[0]);
+                    store_at(f.delx_eta, e, r.delx[1]);
+                    store_at(f.delx_zeta, e, r.delx[2]);
+                }
+                if (r.vnew <= 0.0) {
+                    raise_error(s, -1);
+                }
+            }
+        }
+        if (k + 1 < ke) {
+            fetch_plane(k + 2);
+            store_plane(k + 2);
+        }
+    }
+    if (k1 == nx) {
+        finish(nx - 1, 0.0);  // a free surface above
+    }
+}
+
+// 16 x 16: the tile whose surrounding gradients are exactly one wave's
+constexpr int kLimitTX = 16, kLimitTY = 16;
+
+__global__ __launch_bounds__(kLimitTX *kLimitTY, 3) void k_kinematics_limit(DevFields f, DevScalars *s,
+                                                                         PhysParams prm, int nz,
+                                                                         int store)
+{
+    __shared__ int skip;
+    if (threadIdx.x == 0) {
+        skip = (s->active == 0 || s->error != 0) ? 1 : 0;
+    }
+    __syncthreads();
+    if (skip) {
+        return;
+    }
+    const int nbx = (f.nx + kLimitTX - 1) / kLimitTX, nby = (f.nx + kLimitTY - 1) / kLimitTY;
+    const int tiles = nbx * nby * ((f.nx + nz - 1) / nz);
+    const int t = xcd_order(int(blockIdx.x), tiles);
+    if (t >= tiles) {
+        return;
+    }
+    const int r = t / nbx, bz = r / nby;
+    kinematics_limit_tile<kLimitTX, kLimitTY>(f, s, prm, nz, store != 0, t - r * nbx,
+                                              r - bz * nby, bz);
+}
+
+}  // namespace
+
+int kinematics_limit_columns(int nx)
+{
+    return ((nx + kLimitTX - 1) / kLimitTX) * ((nx + kLimitTY - 1) / kLimitTY);
+}
+
+hipError_t launch_kinematics_limit(const DevFields &f, DevScalars *s, const PhysParams &prm,
+                                   int nz, bool store, hipStream_t stream)
+{
+    if (nz < 1) {
+        return hipErrorInvalidValue;
+    }
+    const int64_t tiles = int64_t(kinematics_limit_columns(f.nx)) * ((f.nx + nz - 1) / nz);
+    hipLaunchKernelGGL(k_kinematics_limit, dim3(unsigned((tiles + 7) / 8 * 8)),
+                       dim3(kLimitTX * kLimitTY), 0, stream, f, s, prm, nz, store ? 1 : 0);
+    return hipGetLastError();
+}
+
+// EOS, volume update and time constraints after k_kinematics_limit, as
+// k_q_eos_dt_nat has them after its limiter.
+__global__ __launch_bounds__(256) void k_eos_dt_nat(DevFields f, DevScalars *s, PhysParams prm)
+{
+    __shared__ unsigned long long lds_c[4], lds_h[4];
+    __shared__ int skip;
+    __shared__ RepLds rep_lds;
+    if (threadIdx.x == 0) {
+        skip = (s->active == 0 || s->error != 0) ? 1 : 0;
+    }
+    __syncthreads();
+    if (skip) {
+        return;
+    }
+    __builtin_amdgcn_s_setprio(1);  // the element's loads first
+    const int el = f.eos_blocks[blockIdx.x] * int(blockDim.x) + int(threadIdx.x);
+    const bool valid = el < f.num_elem;
+    QInputs in;
+    EosIn a{1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int extra = 0;
+    if (valid) {
+        extra = int(f.rep[el]) - 1;
+        const unsigned e = unsigned(el);
+        const double qlin = load_at(f.ql, e), qquad = load_at(f.qq, e);
+        in.vdov = load_at(f.vdov, e);
+        in.vnew = load_at(f.vnew, e);
+        in.q_old = load_at(f.q, e);
+        in.v_old = load_at(f.v, e);
+        in.e_old = load_at(f.e, e);
+        in.p_old = load_at(f.p, e);
+        in.delv = in.vnew - in.v_old;
+        in.arealg = (in.vdov != 0.) ? load_at(f.arealg, e) : 0.0;
+        a = eos_prepare(s, prm, in, qlin, qquad);
+    }
+    eos_nat_block(f, s, prm, el, valid, in, a, extra, lds_c, lds_h, rep_lds);
+}
+#endif  // LULESH_FUSED
 
 // persistent blocks over the element chunks of all members; a chunk lies
 // inside one member, so its minima go to that member's accumulators

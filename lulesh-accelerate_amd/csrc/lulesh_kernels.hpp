@@ -52,6 +52,7 @@ struct DevScalars {
     int error;         // 0, -1 VolumeError, -2 QStopError
     int dt_pending;  // the accumulators hold minima not yet applied
     int cur;         // copy of the node arrays holding the state
+    int last;        // 1 when the run ends with this cycle
 };
 
 // Constants of the method (reference/C/LULESH-OMP.cc:3063-3087;
@@ -544,6 +545,12 @@ __global__ void k_device_math(int op, int n, const double *a, const double *b,
 hipError_t launch_force_sweep(const SweepShape &shape, const DevFields &f,
                               DevScalars *s, const PhysParams &prm,
                               hipStream_t stream);
+// kinematics and the limiter in one sweep, and the EOS that follows it; store:
+// whether the cycle leaves its intermediate fields in memory
+int kinematics_limit_columns(int nx);  // its blocks per chunk of layers
+hipError_t launch_kinematics_limit(const DevFields &f, DevScalars *s, const PhysParams &prm,
+                                   int nz, bool store, hipStream_t stream);
+__global__ void k_eos_dt_nat(DevFields f, DevScalars *s, PhysParams prm);
 __global__ void k_kinematics_q_batch(const BatchMember *members,
                                      const BatchWork *work, PhysParams prm);
 __global__ void k_q_eos_dt_batch(const BatchMember *members, const BatchWork *work,

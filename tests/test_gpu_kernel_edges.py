@@ -51,3 +51,24 @@ def test_fused_step_at_tile_edges(lulesh_gpu, nx, mode):
         assert np.max(np.abs(x - y)) <= 1e-10 * s, f
     a.close()
     b.close()
+
+
+# the sweep of kinematics and limiter serves domains beyond the last-level
+# cache: tiles of 16 x 16 columns, full, one column over and one short
+@pytest.mark.parametrize("nx,mode,step,limit", [(104, 2, 3, None), (112, 1, 2, None),
+                                                (113, 2, 35, None), (127, 2, 40, 33)])
+def test_limiter_sweep_is_the_separate_kernels(lulesh_gpu, nx, mode, step, limit):
+    """Bit for bit the fused step whose kinematics and limiter are separate
+    kernels (the region-sorted schedule), in every field, also those that
+    only a call's last cycle stores: a call that ends inside a replayed
+    graph's length, past it, and at the cycle limit before its own end."""
+    more = {} if limit is None else {"max_cycles": limit}
+    a = lulesh_gpu.Domain(nx, ic_mode=mode, fused=True, **more)
+    b = lulesh_gpu.Domain(nx, ic_mode=mode, fused=True, **more)
+    b.set_eos_bands(1)
+    assert a.step(step) == b.step(step)
+    bad = [f for f in NODE + ELEM
+           if not np.array_equal(a.get(f).view(np.uint64), b.get(f).view(np.uint64))]
+    assert bad == []
+    a.close()
+    b.close()
