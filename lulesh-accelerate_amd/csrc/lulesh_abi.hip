@@ -40,10 +40,9 @@ const char *const kKernelNames[KID_COUNT] = {
     "k_dt_finish", "k_forces_u_blocks", "k_nodes_u",
 };
 
-// default launch shape of the force sweep (32 x 8 element columns, at most
-// 17 node planes per block, register budget for 2 waves per SIMD; the planes
-// per block shrink on small domains, see default_sweep_planes);
-// lulesh_set_sweep_shape overrides it
+// default launch shape of the force sweep: 32 x 8 element columns, register
+// budget for 2 waves per SIMD; the planes per block follow the domain
+// (default_sweep_planes).  lulesh_set_sweep_shape overrides it.
 constexpr SweepShape kDefaultSweep = {32, 8, 17, 2};
 // the mixed-precision sweep holds float32 corner forces: three blocks fit
 // on a CU
@@ -56,46 +55,24 @@ constexpr int kBatch = 32;  // cycles queued per host round trip in run()
 // as often as it fits and queues the rest one launch at a time
 constexpr int kGraphCycles = 32;
 
-// Node planes per block of the default sweep on an nx^3 domain: the largest
-// nz <= 17 whose grid still fills 90% of the resident block slots (two
-// 256-thread blocks per CU).  A block sweeps its planes one after another,
-// so on small domains parallelism comes from cutting the columns into
-// short runs: at 30^3 nz = 1 takes the cycle from 138 to 45 us, at 64^3
-// nz = 4 from 162 to 95 us; from 120^3 on nz = 17 is kept (at 150^3 it
-// runs 0.4% faster than 16: 990 blocks instead of 1100; measured on
-// MI355X).
-int default_sweep_planes(int nx)
-{
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
-            hipSuccess ||
-        cus < 1) {
-        cus = 256;
-    }
-    const long long want = (long long)(0.9 * 2 * cus);
-    const int en = nx + 1;
-    const long long cols = (long long)((en + kDefaultSweep.tx - 2) / (kDefaultSweep.tx - 1)) *
-                           ((en + kDefaultSweep.ty - 2) / (kDefaultSweep.ty - 1));
-    for (int nz = kDefaultSweep.nz; nz > 1; --nz) {
-        if (cols * ((en + nz - 1) / nz) >= want) {
-            return nz;
-        }
-    }
-    return 1;
-}
-
 // Planes (or layers) per block of a sweep that cuts `planes` of them into
 // chunks, `cols` blocks each, `resident` of which a CU holds.  A block takes
 // its planes one after another, so a launch lasts as many rounds of the
 // resident slots as it has, times a block's planes and the `extra` it costs
 // to start (the recomputed halo planes, and about two more for the first
 // loads).  The fewest plane times win, the longer chunk of two equals: its
-// halo is a smaller part.  For the kinematics sweep it picks the
-// fastest of a scan at 150^3 (10 layers, 1.95 rounds, 133 us; 9: 157 us) and
-// 180^3 (12, 2.8 rounds, 225 us; 30: 286 us).
-int plan_planes(int planes, long long cols, int resident, int extra, int most)
+// halo is a smaller part.  In scans over 1 to 61 planes at 64^3 to 240^3 it
+// picks the fastest float64 count, and a mixed one within 2% of it: fused
+// force sweep 120^3 18 planes, 0.98 rounds, 74 us (17 planes: 1.12 rounds,
+// 110 us), 150^3 17, 1.93 rounds, 143 us (16: 2.15, 175 us); bit-identical
+// 91^3 8, 75 us (9: 82 us), 120^3 18, 157 us (17: 234 us); mixed 100^3 9, 70
+// us (8: 103 us, 12: 84 us), 120^3 13, 97 us (12: 144 us); kinematics sweep
+// 150^3 10 layers, 1.95 rounds, 133 us (9: 157 us).  For blocks dispatched
+// in xcd_order: each XCD runs its part out, and the short last chunks of the
+// columns end up together.
+int plan_planes(int planes, long long cols, int resident, int extra)
 {
+    constexpr int most = 64;
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
@@ -115,6 +92,17 @@ int plan_planes(int planes, long long cols, int resident, int extra, int most)
         }
     }
     return best;
+}
+
+// the default sweep's node planes per block on an nx^3 domain: blocks of
+// sh.tx x sh.ty columns, one recomputed layer
+int default_sweep_planes(const SweepShape &sh, int nx, bool mixed)
+{
+    const int en = nx + 1;
+    const long long cols = (long long)((en + sh.tx - 2) / (sh.tx - 1)) *
+                           ((en + sh.ty - 2) / (sh.ty - 1));
+    // blocks a CU holds: 2 of the float64 sweeps, 3 of the mixed one
+    return plan_planes(en, cols, mixed ? 3 : 2, 3);
 }
 
 // Whether the fused step's kinematics and limiter run as one sweep.  The
@@ -617,11 +605,11 @@ int create_domain(const lulesh_config *cfg, bool mixed, double efactor,
     d->cfg = *cfg;
     d->mixed = mixed;
     d->sweep = mixed ? kDefaultSweepMixed : kDefaultSweep;
-    if (!mixed && cfg->nx >= 1 && cfg->nx <= 600) {
+    if (cfg->nx >= 1 && cfg->nx <= 600) {
         const int64_t nx = cfg->nx;
-        d->sweep.nz = default_sweep_planes(cfg->nx);
+        d->sweep.nz = default_sweep_planes(d->sweep, cfg->nx, mixed);
         d->limit_sweep = limiter_in_sweep(nx * nx * nx, (nx + 1) * (nx + 1) * (nx + 1));
-        d->limit_planes = plan_planes(cfg->nx, fused::kinematics_limit_columns(cfg->nx), 3, 5, 64);
+        d->limit_planes = plan_planes(cfg->nx, fused::kinematics_limit_columns(cfg->nx), 3, 5);
     }
     HostMesh m;
     try {

@@ -413,24 +413,30 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f, DevSca
     }
 }
 
+// tiles in the order of k_force_sweep, whose reason holds here too
 template <int TX, int TY, int W>
 __global__ __launch_bounds__(TX *TY, W) void k_force_sweep_mixed(DevFieldsMixed f,
                                                               DevScalars *s,
                                                               PhysParams prm, int nz)
 {
-    sweep_tile_mixed<TX, TY>(f, s, prm, nz, int(blockIdx.x), int(blockIdx.y),
-                             int(blockIdx.z));
+    const int nbx = (f.nx + TX - 1) / (TX - 1), nby = (f.nx + TY - 1) / (TY - 1);
+    const int tiles = nbx * nby * ((f.nx + nz) / nz);
+    const int t = xcd_order(int(blockIdx.x), tiles);
+    if (t >= tiles) {
+        return;
+    }
+    const int r = t / nbx, bz = r / nby;
+    sweep_tile_mixed<TX, TY>(f, s, prm, nz, t - r * nbx, r - bz * nby, bz);
 }
 
 template <int TX, int TY, int W>
 hipError_t launch_mixed_shape(int nz, const DevFieldsMixed &f, DevScalars *s,
                               const PhysParams &prm, hipStream_t stream)
 {
-    const int en = f.nx + 1;
-    const dim3 grid((en + TX - 2) / (TX - 1), (en + TY - 2) / (TY - 1),
-                    (en + nz - 1) / nz);
-    hipLaunchKernelGGL((k_force_sweep_mixed<TX, TY, W>), grid, dim3(TX * TY), 0, stream,
-                       f, s, prm, nz);
+    const int64_t tiles = int64_t((f.nx + TX - 1) / (TX - 1)) *
+                          ((f.nx + TY - 1) / (TY - 1)) * ((f.nx + nz) / nz);
+    hipLaunchKernelGGL((k_force_sweep_mixed<TX, TY, W>), dim3(unsigned((tiles + 7) / 8 * 8)),
+                       dim3(TX * TY), 0, stream, f, s, prm, nz);
     return hipGetLastError();
 }
 

@@ -72,3 +72,21 @@ def test_limiter_sweep_is_the_separate_kernels(lulesh_gpu, nx, mode, step, limit
     assert bad == []
     a.close()
     b.close()
+
+
+# tiles in XCD order: fewer than eight, a multiple of eight and not; the last
+# chunk of the columns whole and short
+@pytest.mark.parametrize("nx,planes", [(1, 1), (5, 2), (31, 7), (61, 64), (62, 20)])
+@pytest.mark.parametrize("mode", ["exact", "fused", "mixed"])
+def test_planes_per_block_change_no_bits(lulesh_gpu, nx, planes, mode):
+    """A domain swept with the planes per block of its own choice against
+    one with the given number: each element's and each node's arithmetic is
+    the same whichever block does it."""
+    a = lulesh_gpu.Domain(nx, fused=mode == "fused", mixed=mode == "mixed")
+    b = lulesh_gpu.Domain(nx, fused=mode == "fused", mixed=mode == "mixed")
+    b.set_sweep_shape(32, 8, planes, 3 if mode == "mixed" else 2)
+    assert a.step(20) == b.step(20)
+    bad = [f for f in NODE + ELEM if not np.array_equal(a.get(f), b.get(f))]
+    assert bad == []
+    a.close()
+    b.close()
