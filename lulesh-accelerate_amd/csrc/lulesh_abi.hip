@@ -298,6 +298,8 @@ int queue_cycle(lulesh_domain *d, bool store)
     DevScalars *s = d->s;
     const DevFields &f = d->f;
     const DevFieldsMixed &fm = d->fm;
+    const int eos_elems = d->mixed ? fm.eos_elems : f.eos_elems;
+    const unsigned gq = unsigned((d->num_elem + eos_elems - 1) / eos_elems);
     const PhysParams &p = d->prm;
     const bool mixed = d->mixed;
     int rc;
@@ -322,7 +324,7 @@ int queue_cycle(lulesh_domain *d, bool store)
              })))
             return rc;
         return launch(d, KID_Q_EOS_DT, [&] {
-            hipLaunchKernelGGL(fused::k_eos_dt_nat, dim3(ge), dim3(kBlock), 0, st, f, s, p);
+            hipLaunchKernelGGL(fused::k_eos_dt_nat, dim3(gq), dim3(kBlock), 0, st, f, s, p);
         });
     }
     if ((rc = launch(d, KID_KINEMATICS_Q, [&] {
@@ -339,7 +341,7 @@ int queue_cycle(lulesh_domain *d, bool store)
         return rc;
     if ((rc = launch(d, KID_Q_EOS_DT, [&] {
              if (mixed && d->eos_bands == 0) {
-                 hipLaunchKernelGGL(k_q_eos_dt_mixed_nat, dim3(ge), dim3(kBlock), 0, st, fm,
+                 hipLaunchKernelGGL(k_q_eos_dt_mixed_nat, dim3(gq), dim3(kBlock), 0, st, fm,
                                     s, p);
              } else if (mixed) {
                  hipLaunchKernelGGL(k_q_eos_dt_mixed, dim3(ge), dim3(kBlock), 0, st, fm, s,
@@ -349,7 +351,7 @@ int queue_cycle(lulesh_domain *d, bool store)
                                     dim3(ge), dim3(kBlock), 0, st, f, s, p, d->learned,
                                     d->learned_z_max, d->learned_form);
              } else if (d->eos_bands == 0) {
-                 hipLaunchKernelGGL(fused ? fused::k_q_eos_dt_nat : k_q_eos_dt_nat, dim3(ge),
+                 hipLaunchKernelGGL(fused ? fused::k_q_eos_dt_nat : k_q_eos_dt_nat, dim3(gq),
                                     dim3(kBlock), 0, st, f, s, p);
              } else {
                  hipLaunchKernelGGL(fused ? fused::k_q_eos_dt : k_q_eos_dt, dim3(ge),

@@ -888,11 +888,10 @@ __device__ __forceinline__ void eos_nat_block(const F &f, DevScalars *s, const P
 // The limiter and the EOS of such a block.
 template <class F>
 __device__ __forceinline__ void q_eos_dt_nat_block(const F &f, DevScalars *s,
-                                                   const PhysParams &prm, int el,
+                                                   const PhysParams &prm, int el, bool valid,
                                                    unsigned long long *lds_c,
                                                    unsigned long long *lds_h, RepLds &L)
 {
-    const bool valid = el < f.num_elem;
     QInputs in;
     EosIn a{1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     int extra = 0;
@@ -914,9 +913,10 @@ __device__ __forceinline__ void q_eos_dt_nat_block(const F &f, DevScalars *s,
 }  // namespace
 
 // Monotonic Q, EOS, volume update and time constraints with the elements in
-// mesh order, one per thread: each block takes 256 consecutive elements, so
-// the limiter's neighbour values and the element's own fields are read in
-// the order they lie in memory.  The regions' EOS repetitions are shared
+// mesh order, one per thread: each block takes f.eos_elems consecutive
+// elements (256, on small domains fewer; eos_block_elems), so the limiter's
+// neighbour values and the element's own fields are read in the order they
+// lie in memory.  The regions' EOS repetitions are shared
 // over each block's threads (eos_extra_evaluations), and the blocks run in
 // the order f.eos_blocks gives (costliest first, then the rest in mesh
 // order, each XCD on one contiguous part of the mesh; eos_block_order).
@@ -934,9 +934,9 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_nat(DevFields f, DevScalars *s
         return;
     }
     __builtin_amdgcn_s_setprio(1);  // the element's loads first
-    const int b = f.eos_blocks[blockIdx.x];
-    q_eos_dt_nat_block(f, s, prm, b * int(blockDim.x) + int(threadIdx.x), lds_c, lds_h,
-                       rep_lds);
+    const int el = f.eos_blocks[blockIdx.x] * f.eos_elems + int(threadIdx.x);
+    q_eos_dt_nat_block(f, s, prm, el, int(threadIdx.x) < f.eos_elems && el < f.num_elem, lds_c,
+                       lds_h, rep_lds);
 }
 
 #ifdef LULESH_FUSED
@@ -1244,8 +1244,8 @@ __global__ __launch_bounds__(256) void k_eos_dt_nat(DevFields f, DevScalars *s, 
         return;
     }
     __builtin_amdgcn_s_setprio(1);  // the element's loads first
-    const int el = f.eos_blocks[blockIdx.x] * int(blockDim.x) + int(threadIdx.x);
-    const bool valid = el < f.num_elem;
+    const int el = f.eos_blocks[blockIdx.x] * f.eos_elems + int(threadIdx.x);
+    const bool valid = int(threadIdx.x) < f.eos_elems && el < f.num_elem;
     QInputs in;
     EosIn a{1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     int extra = 0;
@@ -1289,8 +1289,9 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_batch(const BatchMember *__res
             continue;
         }
         __builtin_amdgcn_s_setprio(1);  // the element's loads first
-        q_eos_dt_nat_block(global_view(m.f), m.s, prm, chunks[2 * c + 1] + int(threadIdx.x),
-                           lds_c, lds_h, rep_lds);
+        const int el = chunks[2 * c + 1] + int(threadIdx.x);
+        q_eos_dt_nat_block(global_view(m.f), m.s, prm, el, el < m.f.num_elem, lds_c, lds_h,
+                           rep_lds);
     }
 }
 
@@ -1315,8 +1316,8 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_chunks(const BatchMember *__re
         return;
     }
     __builtin_amdgcn_s_setprio(1);  // the element's loads first
-    q_eos_dt_nat_block(global_view(m.f), m.s, prm, chunks[2 * c + 1] + int(threadIdx.x),
-                       lds_c, lds_h, rep_lds);
+    const int el = chunks[2 * c + 1] + int(threadIdx.x);
+    q_eos_dt_nat_block(global_view(m.f), m.s, prm, el, el < m.f.num_elem, lds_c, lds_h, rep_lds);
 }
 
 // ---------------------------------------------------------------------------

@@ -119,6 +119,7 @@ struct DevFields {
     // the EOS evaluations beyond an element's first, in its light and in its
     // costly regions: the two values that repetitions - 1 takes besides 0
     int eos_extra[2];
+    int eos_elems;  // elements per block of the mesh-order Q/EOS launch
     FastDiv div_nx;
     // node-centred: positions and velocities in two copies (see above)
     double *x[2], *y[2], *z[2], *xd[2], *yd[2], *zd[2];
@@ -399,7 +400,7 @@ __device__ __forceinline__ bool member_running(const DevScalars *s)
 struct DevFieldsMixed {
     int nx;
     int num_elem, num_node;
-    int eos_extra[2];  // see DevFields
+    int eos_extra[2], eos_elems;  // see DevFields
     FastDiv div_nx;
     double *x[2], *y[2], *z[2], *xd[2], *yd[2], *zd[2];
     double *nodal_mass;

@@ -287,12 +287,15 @@ HostMesh build_mesh(const MeshConfig &cfg)
         std::swap(m.eos_extra[0], m.eos_extra[1]);
     }
     m.eos_blocks = eos_block_order(m.elem_rep);
+    m.eos_elems = eos_block_elems(m.num_elem, m.eos_extra[1] > 0);
+    m.eos_launch = (m.eos_elems == kEosBlockElems) ? m.eos_blocks
+                                                   : eos_block_order(m.elem_rep, m.eos_elems);
     return m;
 }
 
 // A block's cost is its EOS passes: one for the elements' own evaluations,
 // plus the evaluations beyond each element's first shared over the block's
-// threads, ceil(sum(rep - 1) / kEosBlockElems).  With LULESH 2.0's regions
+// threads, ceil(sum(rep - 1) / 256).  With LULESH 2.0's regions
 // the costs are far from even: at 150^3 (cost 1, 11 regions) 8% of the
 // blocks lie in runs of the 20-repetition region and take 20 passes, 40%
 // take 2, the mean is 4.6.  A costly block started late runs on after the
@@ -307,15 +310,38 @@ HostMesh build_mesh(const MeshConfig &cfg)
 // against mesh order alone: 90^3 52.0 -> 38.2 us, 120^3 90.3 -> 75.3 us,
 // 150^3 146.3 -> 140.5 us (float64 with fused multiply-adds); mixed
 // precision 120^3 64.8 -> 54.8 us.
+//
+// One domain alone.  A block of 256 elements inside the 20-repetition region
+// runs 20 evaluations one after another, and on a small domain the cycle
+// waits for it while most CUs have no block.  With fewer elements a block's
+// 256 threads share fewer evaluations.  The line is where the blocks, each
+// of which has one wave or two that load and limit, outnumber what the chip
+// holds and so cost more than they save.  Step time in us with 64, 128 and
+// 256 elements per block (11 regions, bit-identical): 30^3 30.7, 34.0, 39.6;
+// 45^3 48.3, 50.3, 55.9; 55^3 56.0, 56.8, 60.0; 64^3 79.3, 77.2, 81.7; 80^3
+// 117, 110, 108; fused 30^3 22.8, 25.4, 30.3; mixed 25.9, 28.2, 32.5.  32
+// are 0.2 us better to 4 us worse from 30^3 to 45^3.  With one repetition
+// everywhere there is nothing to share (45^3 44.8, 43.9, 43.8).
+int eos_block_elems(int64_t num_elem, bool repeated)
+{
+    constexpr int kLeast = 64;
+    constexpr int64_t kMostBlocks = 2700;
+    int elems = kEosBlockElems;
+    while (repeated && elems > kLeast && num_elem <= kMostBlocks * (elems / 2)) {
+        elems /= 2;
+    }
+    return elems;
+}
+
 namespace {
 
 constexpr double kHeavyCost = 1.0, kHeavySpan = 0.75;
 
 }  // namespace
 
-std::vector<int64_t> eos_block_passes(const std::vector<uint16_t> &rep)
+std::vector<int64_t> eos_block_passes(const std::vector<uint16_t> &rep, int elems)
 {
-    const size_t ne = rep.size(), be = size_t(kEosBlockElems);
+    const size_t ne = rep.size(), be = size_t(elems);
     const size_t g = (ne + be - 1) / be;
     std::vector<int64_t> passes(g);
     for (size_t b = 0; b < g; ++b) {
@@ -323,14 +349,14 @@ std::vector<int64_t> eos_block_passes(const std::vector<uint16_t> &rep)
         for (size_t i = b * be; i < std::min(ne, (b + 1) * be); ++i) {
             extra += int64_t(rep[i]) - 1;
         }
-        passes[b] = 1 + (extra + int64_t(be) - 1) / int64_t(be);
+        passes[b] = 1 + (extra + kEosBlockElems - 1) / kEosBlockElems;
     }
     return passes;
 }
 
-std::vector<int32_t> eos_block_order(const std::vector<uint16_t> &rep)
+std::vector<int32_t> eos_block_order(const std::vector<uint16_t> &rep, int elems)
 {
-    return spread_costly_blocks(eos_block_passes(rep));
+    return spread_costly_blocks(eos_block_passes(rep, elems));
 }
 
 std::vector<int32_t> spread_costly_blocks(const std::vector<int64_t> &passes)

@@ -40,21 +40,29 @@ struct HostMesh {
     std::vector<int32_t> region_offset; // start of each region in eos_order
     std::vector<uint16_t> elem_rep;     // EOS repetitions of each element
     int eos_extra[2] = {0, 0};          // the values of elem_rep - 1 besides 0: light, heavy
-    std::vector<int32_t> eos_blocks;    // dispatch order of the mesh-order Q/EOS blocks
+    std::vector<int32_t> eos_blocks;    // dispatch order of blocks of kEosBlockElems elements
+    int eos_elems = 0;                  // elements per block of a domain's own Q/EOS launch
+    std::vector<int32_t> eos_launch;    // and that launch's order
 };
 
-// Elements per block of the mesh-order Q/EOS kernels (one per thread).
+// Threads, and elements at most, of a block of the mesh-order Q/EOS kernels.
 constexpr int kEosBlockElems = 256;
 
+// The elements of such a block in the launch of one domain, fewer than its
+// threads where the domain is small and has repetitions to share.
+int eos_block_elems(int64_t num_elem, bool repeated);
+
 // The order in which the blocks of a mesh-order Q/EOS launch take the mesh's
-// blocks of kEosBlockElems consecutive elements (eos_block_order in
+// blocks of `elems` consecutive elements (eos_block_order in
 // lulesh_mesh.cpp): slot t of the launch processes block order[t].
-std::vector<int32_t> eos_block_order(const std::vector<uint16_t> &rep);
+std::vector<int32_t> eos_block_order(const std::vector<uint16_t> &rep,
+                                     int elems = kEosBlockElems);
 // Its two parts: the EOS passes of each block (one, plus the evaluations
 // beyond each element's first shared over the block), and the launch order
 // of blocks of the given costs, listed in the order whose locality the
 // launch should keep.
-std::vector<int64_t> eos_block_passes(const std::vector<uint16_t> &rep);
+std::vector<int64_t> eos_block_passes(const std::vector<uint16_t> &rep,
+                                      int elems = kEosBlockElems);
 std::vector<int32_t> spread_costly_blocks(const std::vector<int64_t> &passes);
 
 // Builds the mesh, masses, ICs and regions; throws std::invalid_argument.

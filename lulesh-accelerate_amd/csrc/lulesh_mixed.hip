@@ -962,7 +962,7 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_mixed(DevFieldsMixed f, DevSca
     fold_minima_mixed(s, cand_c, cand_h, lds_c, lds_h);
 }
 
-// Mesh order, one element per thread, blocks of 256 consecutive elements in
+// Mesh order, one element per thread, blocks of f.eos_elems consecutive elements in
 // the order f.eos_blocks gives, the regions' EOS repetitions shared over
 // each block's threads (as k_q_eos_dt_nat).  Each element's arithmetic is
 // that of k_q_eos_dt_mixed, so both give the same bits.
@@ -980,8 +980,8 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_mixed_nat(DevFieldsMixed f, De
         return;
     }
     __builtin_amdgcn_s_setprio(1);  // the element's loads first
-    const int el = f.eos_blocks[blockIdx.x] * int(blockDim.x) + int(threadIdx.x);
-    const bool valid = el < f.num_elem;
+    const int el = f.eos_blocks[blockIdx.x] * f.eos_elems + int(threadIdx.x);
+    const bool valid = int(threadIdx.x) < f.eos_elems && el < f.num_elem;
     const EosConstMixed ec = eos_const_mixed(prm);
     unsigned long long cand_c = as_bits(kBig), cand_h = as_bits(kBig);
     QKeepMixed kp{1.0, 0.f, 0.f};

@@ -53,7 +53,7 @@ size_t domain_arena_bytes(const HostMesh &m)
     const size_t pn = round_up(size_t(m.num_node), 64);
     size_t bytes = (kNodeArrays * pn + kElemArrays * pe) * sizeof(double);
     bytes += round_up(pe * sizeof(int32_t), 256) + 2 * round_up(pe * sizeof(uint16_t), 256);
-    bytes += round_up(m.eos_blocks.size() * sizeof(int32_t), 256);
+    bytes += round_up(m.eos_launch.size() * sizeof(int32_t), 256);
     bytes += round_up(sizeof(DevScalars), 256);
     return bytes;
 }
@@ -71,6 +71,7 @@ void carve_domain(char *base, const HostMesh &m, DevFields &f, DevScalars **s)
     f.div_nx = make_fastdiv(unsigned(m.nx));
     f.eos_extra[0] = m.eos_extra[0];
     f.eos_extra[1] = m.eos_extra[1];
+    f.eos_elems = m.eos_elems;
     for (int c = 0; c < 2; ++c) {
         f.x[c] = take_node(); f.y[c] = take_node(); f.z[c] = take_node();
         f.xd[c] = take_node(); f.yd[c] = take_node(); f.zd[c] = take_node();
@@ -91,7 +92,7 @@ void carve_domain(char *base, const HostMesh &m, DevFields &f, DevScalars **s)
     f.rep = reinterpret_cast<uint16_t *>(sched);
     sched += round_up(pe * sizeof(uint16_t), 256);
     f.eos_blocks = reinterpret_cast<int32_t *>(sched);
-    sched += round_up(m.eos_blocks.size() * sizeof(int32_t), 256);
+    sched += round_up(m.eos_launch.size() * sizeof(int32_t), 256);
     *s = reinterpret_cast<DevScalars *>(sched);
 }
 
@@ -112,8 +113,8 @@ hipError_t upload_mesh(const HostMesh &m, const DevFields &f, hipStream_t stream
         {const_cast<int32_t *>(f.eos_order), m.eos_order.data(), ne * sizeof(int32_t)},
         {const_cast<uint16_t *>(f.eos_rep), m.eos_rep.data(), ne * sizeof(uint16_t)},
         {const_cast<uint16_t *>(f.rep), m.elem_rep.data(), ne * sizeof(uint16_t)},
-        {const_cast<int32_t *>(f.eos_blocks), m.eos_blocks.data(),
-         m.eos_blocks.size() * sizeof(int32_t)},
+        {const_cast<int32_t *>(f.eos_blocks), m.eos_launch.data(),
+         m.eos_launch.size() * sizeof(int32_t)},
     };
     for (const Copy &c : copies) {
         const hipError_t e =
@@ -155,7 +156,7 @@ size_t domain_arena_bytes_mixed(const HostMesh &m)
     size_t bytes = (kNodeArrays * pn + kElemArrays64 * pe) * sizeof(double) +
                    kElemArrays32 * pe * sizeof(float);
     bytes += round_up(pe * sizeof(int32_t), 256) + 2 * round_up(pe * sizeof(uint16_t), 256);
-    bytes += round_up(m.eos_blocks.size() * sizeof(int32_t), 256);
+    bytes += round_up(m.eos_launch.size() * sizeof(int32_t), 256);
     bytes += round_up(sizeof(DevScalars), 256);
     return bytes;
 }
@@ -173,6 +174,7 @@ void carve_domain_mixed(char *base, const HostMesh &m, DevFieldsMixed &f, DevSca
     f.div_nx = make_fastdiv(unsigned(m.nx));
     f.eos_extra[0] = m.eos_extra[0];
     f.eos_extra[1] = m.eos_extra[1];
+    f.eos_elems = m.eos_elems;
     for (int c = 0; c < 2; ++c) {
         f.x[c] = take_node(); f.y[c] = take_node(); f.z[c] = take_node();
         f.xd[c] = take_node(); f.yd[c] = take_node(); f.zd[c] = take_node();
@@ -194,7 +196,7 @@ void carve_domain_mixed(char *base, const HostMesh &m, DevFieldsMixed &f, DevSca
     f.rep = reinterpret_cast<uint16_t *>(sched);
     sched += round_up(pe * sizeof(uint16_t), 256);
     f.eos_blocks = reinterpret_cast<int32_t *>(sched);
-    sched += round_up(m.eos_blocks.size() * sizeof(int32_t), 256);
+    sched += round_up(m.eos_launch.size() * sizeof(int32_t), 256);
     *s = reinterpret_cast<DevScalars *>(sched);
 }
 

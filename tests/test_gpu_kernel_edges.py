@@ -90,3 +90,21 @@ def test_planes_per_block_change_no_bits(lulesh_gpu, nx, planes, mode):
     assert bad == []
     a.close()
     b.close()
+
+
+# Q/EOS blocks of 64 elements up to 55^3, of 128 up to 70^3, of 256 beyond;
+# the last block full (4^3, 64^3), partial and short
+@pytest.mark.parametrize("nx", [4, 5, 55, 56, 57, 64, 70, 71])
+@pytest.mark.parametrize("mode", ["exact", "fused", "mixed"])
+def test_small_q_eos_blocks_change_no_bits(lulesh_gpu, nx, mode):
+    """Against the region-sorted schedule, which shares no evaluations."""
+    a = lulesh_gpu.Domain(nx, fused=mode == "fused", mixed=mode == "mixed")
+    b = lulesh_gpu.Domain(nx, fused=mode == "fused", mixed=mode == "mixed")
+    b.set_eos_bands(1)
+    assert a.step(20) == b.step(20)
+    bad = [f for f in NODE + ELEM if not np.array_equal(a.get(f), b.get(f))]
+    assert bad == []
+    sa, sb = a.stats(), b.stats()
+    assert (sa.time, sa.dtcourant, sa.dthydro) == (sb.time, sb.dtcourant, sb.dthydro)
+    a.close()
+    b.close()
