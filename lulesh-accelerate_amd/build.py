@@ -25,10 +25,11 @@ HARNESS = os.path.join(PKG, "lulesh_mi355x")
 
 HIP_SOURCES = ["lulesh_kernels.hip", "lulesh_force.hip", "lulesh_mixed.hip",
                "lulesh_abi.hip", "lulesh_batch.hip", "lulesh_mlp.hip",
-               "lulesh_setup.cpp", "lulesh_output.cpp",
-               "lulesh_mesh.cpp"]
+               "lulesh_transfer.hip", "lulesh_setup.cpp",
+               "lulesh_output.cpp", "lulesh_mesh.cpp"]
 HEADERS = ["lulesh_kernels.hpp", "lulesh_elem.hpp", "lulesh_modal.hpp", "lulesh_cbrt.h",
-           "lulesh_mesh.hpp", "lulesh_setup.hpp", "lulesh_mlp.hpp"]
+           "lulesh_mesh.hpp", "lulesh_setup.hpp", "lulesh_mlp.hpp",
+           "lulesh_transfer.hpp"]
 # built a second time with multiply-adds fused (namespace lulesh::fused)
 FUSED_SOURCES = ["lulesh_force.hip", "lulesh_kernels.hip"]
 OBJ_DIR = os.path.join(PKG, "_build")

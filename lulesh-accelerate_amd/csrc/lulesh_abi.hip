@@ -19,6 +19,7 @@
 #include "lulesh_mesh.hpp"
 #include "lulesh_mlp.hpp"
 #include "lulesh_setup.hpp"
+#include "lulesh_transfer.hpp"
 
 using namespace lulesh;
 
@@ -137,9 +138,10 @@ struct lulesh_domain {
     DevForceBlocksU fblocks{};  // its element blocks
     int64_t boundary_corners = 0;
     // An unstructured mesh is held renumbered (renumber_mesh_u): the new
-    // number of each element and node of the mesh as given, which the field
-    // copies map, and the nodelist as given ([8][num_elem]).
-    std::vector<int32_t> elem_new, node_new, nodelist_given;
+    // number of each element and node of the mesh as given, on the device,
+    // which the field copies map, and the nodelist as given ([8][num_elem]).
+    const int32_t *elem_place = nullptr, *node_place = nullptr;
+    std::vector<int32_t> nodelist_given;
     int origin = 0;             // the element holding the initial energy
     int origin_dev = 0;         //   and its number on the device
     std::vector<void *> bufs;   // device allocations of an unstructured domain
@@ -156,6 +158,7 @@ struct lulesh_domain {
     int limit_planes = 1;      //   and its element layers per block
     void *arena = nullptr;
     hipStream_t stream = nullptr;
+    FieldTransfer transfer;
 
     bool timing = false;
     std::vector<hipEvent_t> event_pool;
@@ -466,84 +469,20 @@ int collect_timings(lulesh_domain *d)
     return LULESH_OK;
 }
 
-struct FieldRef {
-    void *ptr;
-    int64_t n;
-    bool f32;                  // stored as float32 (mixed precision)
-    const int32_t *renumber;   // device place of each value, or null (in order)
-};
-
-// par: the copy of the node arrays that holds the current state
-FieldRef field_ref(lulesh_domain *d, int id, int par)
+// A field on the device, the host's values of it at `host`.  par: the copy of
+// the node arrays that holds the current state.
+TransferItem field_ref(lulesh_domain *d, int id, int par, double *host)
 {
-    FieldRef r{nullptr, 0, false, nullptr};
+    TransferItem r{nullptr, host, 0, false, nullptr};
     if (d->mixed) {
-        r.ptr = field_pointer_mixed(d->fm, id, par, &r.n, &r.f32);
+        r.dev = field_pointer_mixed(d->fm, id, par, &r.n, &r.f32);
     } else {
-        r.ptr = field_pointer(d->f, id, par, &r.n);
+        r.dev = field_pointer(d->f, id, par, &r.n);
     }
-    if (d->unstructured && r.ptr) {
-        r.renumber = (id < LULESH_F_E) ? d->node_new.data() : d->elem_new.data();
+    if (d->unstructured) {
+        r.place = (id < LULESH_F_E) ? d->node_place : d->elem_place;
     }
     return r;
-}
-
-// host float64 <-> device field (converted when the field is float32, put
-// in the device's order when the mesh is renumbered); synchronous
-int copy_in(lulesh_domain *d, const FieldRef &r, const double *src)
-{
-    if (r.renumber) {
-        std::vector<double> tmp(static_cast<size_t>(r.n));
-        for (int64_t i = 0; i < r.n; ++i) {
-            tmp[size_t(r.renumber[i])] = src[i];
-        }
-        HIP_TRY(d, hipMemcpyAsync(r.ptr, tmp.data(), tmp.size() * sizeof(double),
-                                  hipMemcpyHostToDevice, d->stream));
-        HIP_TRY(d, hipStreamSynchronize(d->stream));
-        return LULESH_OK;
-    }
-    if (!r.f32) {
-        HIP_TRY(d, hipMemcpyAsync(r.ptr, src, size_t(r.n) * sizeof(double),
-                                  hipMemcpyHostToDevice, d->stream));
-        HIP_TRY(d, hipStreamSynchronize(d->stream));
-        return LULESH_OK;
-    }
-    std::vector<float> tmp(static_cast<size_t>(r.n));
-    for (int64_t i = 0; i < r.n; ++i) {
-        tmp[size_t(i)] = static_cast<float>(src[i]);
-    }
-    HIP_TRY(d, hipMemcpyAsync(r.ptr, tmp.data(), tmp.size() * sizeof(float),
-                              hipMemcpyHostToDevice, d->stream));
-    HIP_TRY(d, hipStreamSynchronize(d->stream));
-    return LULESH_OK;
-}
-
-int copy_out(lulesh_domain *d, double *dst, const FieldRef &r)
-{
-    if (r.renumber) {
-        std::vector<double> tmp(static_cast<size_t>(r.n));
-        HIP_TRY(d, hipMemcpyAsync(tmp.data(), r.ptr, tmp.size() * sizeof(double),
-                                  hipMemcpyDeviceToHost, d->stream));
-        HIP_TRY(d, hipStreamSynchronize(d->stream));
-        for (int64_t i = 0; i < r.n; ++i) {
-            dst[i] = tmp[size_t(r.renumber[i])];
-        }
-        return LULESH_OK;
-    }
-    if (!r.f32) {
-        HIP_TRY(d, hipMemcpyAsync(dst, r.ptr, size_t(r.n) * sizeof(double),
-                                  hipMemcpyDeviceToHost, d->stream));
-        HIP_TRY(d, hipStreamSynchronize(d->stream));
-        return LULESH_OK;
-    }
-    std::vector<float> tmp(static_cast<size_t>(r.n));
-    HIP_TRY(d, hipMemcpyAsync(tmp.data(), r.ptr, tmp.size() * sizeof(float),
-                              hipMemcpyDeviceToHost, d->stream));
-    HIP_TRY(d, hipStreamSynchronize(d->stream));
-    for (int64_t i = 0; i < r.n; ++i) {
-        dst[i] = static_cast<double>(tmp[size_t(i)]);
-    }
-    return LULESH_OK;
 }
 
 // the domain tuple's fields in the order of upload/download_state
@@ -748,6 +687,10 @@ int build_device_domain_u(lulesh_domain *d, const HostMeshU &m, const ForceBlock
     uint8_t *sy = nullptr;
     if ((rc = upload_vec(d, m.symm, &sy))) return rc;
     g.symm = sy;
+    if ((rc = upload_vec(d, fb.elem_new, &a))) return rc;
+    d->elem_place = a;
+    if ((rc = upload_vec(d, fb.node_new, &a))) return rc;
+    d->node_place = a;
     // the element blocks of the force kernel, and the slots of the boundary
     // nodes' corner forces
     DevForceBlocksU &b = d->fblocks;
@@ -825,8 +768,6 @@ int create_domain_u(const MeshLists &lists, const lulesh_config *cfg, lulesh_dom
     d->reg_num_list.assign(size_t(m.num_elem), 1);
     d->origin = given.origin;
     d->origin_dev = m.origin;
-    d->elem_new = fb.elem_new;
-    d->node_new = fb.node_new;
     d->nodelist_given = std::move(given.nodelist);
     d->prm = make_params(LULESH_IC_1_0);
     if (hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking) != hipSuccess) {
@@ -1050,9 +991,11 @@ int lulesh_upload_state(lulesh_domain *d, const double *x, const double *y,
     int rc = read_scalars(d, &s);
     if (rc) return rc;
     const double *src[11] = {x, y, z, xd, yd, zd, e, p, q, v, ss};
+    TransferItem items[11];
     for (int i = 0; i < 11; ++i) {
-        if ((rc = copy_in(d, field_ref(d, kStateFields[i], s.cur), src[i]))) return rc;
+        items[i] = field_ref(d, kStateFields[i], s.cur, const_cast<double *>(src[i]));
     }
+    HIP_TRY(d, d->transfer.run(items, 11, true, d->stream));
     return lulesh_set_scalars(d, &time, &deltatime, nullptr, nullptr, nullptr);
 }
 
@@ -1068,9 +1011,11 @@ int lulesh_download_state(lulesh_domain *d, double *x, double *y, double *z,
     int rc = read_scalars(d, &s);
     if (rc) return rc;
     double *dst[11] = {x, y, z, xd, yd, zd, e, p, q, v, ss};
+    TransferItem items[11];
     for (int i = 0; i < 11; ++i) {
-        if ((rc = copy_out(d, dst[i], field_ref(d, kStateFields[i], s.cur)))) return rc;
+        items[i] = field_ref(d, kStateFields[i], s.cur, dst[i]);
     }
+    HIP_TRY(d, d->transfer.run(items, 11, false, d->stream));
     if (time) *time = s.time;
     if (deltatime) *deltatime = s.deltatime;
     return LULESH_OK;
@@ -1084,11 +1029,12 @@ int lulesh_get_field(lulesh_domain *d, int field, double *host_out)
     DevScalars s{};
     int rc = read_scalars(d, &s);
     if (rc) return rc;
-    const FieldRef r = field_ref(d, field, s.cur);
-    if (!r.ptr) {
+    const TransferItem r = field_ref(d, field, s.cur, host_out);
+    if (!r.dev) {
         return fail(d, LULESH_BAD_ARG, "unknown field id");
     }
-    return copy_out(d, host_out, r);
+    HIP_TRY(d, d->transfer.run(&r, 1, false, d->stream));
+    return LULESH_OK;
 }
 
 int lulesh_set_field(lulesh_domain *d, int field, const double *host_in)
@@ -1099,11 +1045,12 @@ int lulesh_set_field(lulesh_domain *d, int field, const double *host_in)
     DevScalars s{};
     int rc = read_scalars(d, &s);
     if (rc) return rc;
-    const FieldRef r = field_ref(d, field, s.cur);
-    if (!r.ptr) {
+    const TransferItem r = field_ref(d, field, s.cur, const_cast<double *>(host_in));
+    if (!r.dev) {
         return fail(d, LULESH_BAD_ARG, "unknown field id");
     }
-    return copy_in(d, r, host_in);
+    HIP_TRY(d, d->transfer.run(&r, 1, true, d->stream));
+    return LULESH_OK;
 }
 
 int lulesh_get_stats(lulesh_domain *d, lulesh_stats *out)

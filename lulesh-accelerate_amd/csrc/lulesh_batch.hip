@@ -28,6 +28,7 @@
 #include "lulesh_kernels.hpp"
 #include "lulesh_mesh.hpp"
 #include "lulesh_setup.hpp"
+#include "lulesh_transfer.hpp"
 
 using namespace lulesh;
 
@@ -85,6 +86,7 @@ struct lulesh_batch {
     int cu_count = 256;
 
     hipStream_t stream = nullptr;
+    FieldTransfer transfer;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     bool graph_stale = true;
@@ -606,9 +608,8 @@ int lulesh_batch_get_field(lulesh_batch *b, int member, int field, double *host_
     if (!p) {
         return bfail(b, LULESH_BAD_ARG, "unknown field id");
     }
-    BHIP_TRY(b, hipMemcpyAsync(host_out, p, size_t(count) * sizeof(double),
-                               hipMemcpyDeviceToHost, b->stream));
-    BHIP_TRY(b, hipStreamSynchronize(b->stream));
+    const TransferItem t{const_cast<double *>(p), host_out, count, false, nullptr};
+    BHIP_TRY(b, b->transfer.run(&t, 1, false, b->stream));
     return LULESH_OK;
 }
 

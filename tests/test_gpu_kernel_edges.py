@@ -108,3 +108,30 @@ def test_small_q_eos_blocks_change_no_bits(lulesh_gpu, nx, mode):
     assert (sa.time, sa.dtcourant, sa.dthydro) == (sb.time, sb.dtcourant, sb.dthydro)
     a.close()
     b.close()
+
+
+# one thread below 4 MB in all (8^3, 29^3), several beyond; fields of one slot
+# (4 MB) and of more: the elements of 80^3 in one, its nodes in two
+@pytest.mark.parametrize("nx,mode", [(1, "exact"), (8, "exact"), (29, "exact"), (37, "exact"),
+                                     (80, "exact"), (128, "exact"), (8, "mixed"),
+                                     (37, "mixed"), (101, "mixed"), (8, "mesh"),
+                                     (37, "mesh"), (81, "mesh")])
+def test_state_there_and_back(lulesh_gpu, oracle, nx, mode):
+    """Every value of a state is found in its place, with the state and by
+    field; values that float32 holds."""
+    if mode == "mesh":
+        d = lulesh_gpu.Domain.from_mesh(oracle.cube_mesh(nx), max_cycles=5)
+    else:
+        d = lulesh_gpu.Domain(nx, mixed=mode == "mixed")
+    st = {"time": 0.25, "deltatime": 0.125}
+    for t, f in enumerate(("x", "y", "z", "xd", "yd", "zd", "e", "p", "q", "v", "ss")):
+        n = d.num_node if t < 6 else d.num_elem
+        st[f] = np.arange(n, dtype=np.float64) + 7 * t
+    d.upload_state(st)
+    back = d.download_state()
+    assert all(np.array_equal(back[f], st[f]) for f in st)
+    for f in ("z", "ss"):
+        assert np.array_equal(d.get(f), st[f])
+        d.set(f, st[f][::-1].copy())
+        assert np.array_equal(d.get(f), st[f][::-1])
+    d.close()
