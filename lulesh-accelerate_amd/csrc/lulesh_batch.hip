@@ -34,9 +34,9 @@ using namespace lulesh;
 
 namespace {
 
-// the autotuner's pick on the 64-member ensemble of nx 16..64 (16 x 8
-// columns, 16 planes, one block per tile and per chunk): 2.84 s to t = 1e-2
-// against 2.97 s for 32 x 8, measured on MI355X
+// 16 x 8 columns, one block per tile and per chunk, the planes by plan_planes:
+// runs of 64 members of 16^3 to 64^3 2.09 s (32 x 8 columns 2.23 s), of 32
+// members of 12^3 to 44^3 240 ms (281 ms)
 constexpr SweepShape kDefaultBatchSweep = {16, 8, 16, 2};
 constexpr int kDefaultCyclesPerGraph = 16;
 constexpr int kTimeBlock = 256;
@@ -75,15 +75,20 @@ struct lulesh_batch {
     std::vector<int4> tiles;
     std::vector<int2> chunks;
     std::vector<int2> eos_chunks;
-    std::vector<std::vector<int64_t>> eos_passes;  // EOS passes of each member's chunks
+    // the EOS evaluations beyond each element's first, of every
+    // kEosBlockLeast elements of each member
+    std::vector<std::vector<int32_t>> eos_extra;
     std::vector<char> dropped;  // members no longer in the work lists
     int full_tiles = 0, full_chunks = 0;
+    size_t tiles_room = 0, eos_room = 0;  // entries of d_tiles, d_eos_chunks
 
     SweepShape sweep = kDefaultBatchSweep;
+    bool plan = true;  // sweep.nz follows the work left, until lulesh_batch_set_shape
     int sweep_blocks = 0, elem_blocks = 0;
     bool fused = false;  // the phases of lulesh::fused (lulesh_batch_set_fused_multiply_add)
     int cycles_per_graph = kDefaultCyclesPerGraph;
     int cu_count = 256;
+    int eos_elems = kChunk;  // elements per Q/EOS chunk
 
     hipStream_t stream = nullptr;
     FieldTransfer transfer;
@@ -125,16 +130,30 @@ int bfail(lulesh_batch *b, int code, const std::string &msg)
 static_assert(kChunk == kEosBlockElems, "a Q/EOS chunk is one Q/EOS block");
 void order_eos_chunks(lulesh_batch *b, bool all)
 {
+    int64_t elems = 0;
+    bool repeated = false;
+    for (int m = 0; m < b->n; ++m) {
+        if (all || !b->dropped[m]) {
+            elems += b->f[m].num_elem;
+            repeated = repeated || b->f[m].eos_extra[1] > 0;
+        }
+    }
+    b->eos_elems = eos_block_elems(elems, repeated);
+    const size_t per = size_t(b->eos_elems / kEosBlockLeast);
     std::vector<int2> base;
     std::vector<int64_t> passes;
     for (int m = 0; m < b->n; ++m) {
         if (!all && b->dropped[m]) {
             continue;
         }
-        const std::vector<int64_t> &p = b->eos_passes[size_t(m)];
-        for (size_t c = 0; c < p.size(); ++c) {
-            base.push_back(make_int2(m, int(c) * kChunk));
-            passes.push_back(p[c]);
+        const std::vector<int32_t> &x = b->eos_extra[size_t(m)];
+        for (size_t c = 0; c < x.size(); c += per) {
+            int64_t extra = 0;
+            for (size_t i = c; i < std::min(x.size(), c + per); ++i) {
+                extra += x[i];
+            }
+            base.push_back(make_int2(m, int(c) * kEosBlockLeast));
+            passes.push_back(1 + (extra + kChunk - 1) / kChunk);
         }
     }
     const std::vector<int32_t> order = spread_costly_blocks(passes);
@@ -144,12 +163,51 @@ void order_eos_chunks(lulesh_batch *b, bool all)
     }
 }
 
+// Node planes per tile for the members in the lists: the sweep's time is the
+// number of rounds its tiles make of the resident blocks (waves per SIMD
+// over waves per block, on four SIMDs) times a tile's planes and what it
+// costs to start, three more.  As members stop, the few that are left are
+// cut finer.  Against 16 planes throughout, with the finer Q/EOS chunks and
+// the tiles in XCD order: runs of 32 members of 12^3 to 44^3 294 -> 240 ms
+// (fused 246 -> 150), of 4 members of 20^3 to 40^3 168 -> 85 ms, of 64
+// members of 16^3 to 64^3 2.10 -> 2.09 s (fused 1.84 -> 1.41).
+int plan_planes(const lulesh_batch *b, bool all)
+{
+    if (!all && std::find(b->dropped.begin(), b->dropped.end(), 0) == b->dropped.end()) {
+        return b->sweep.nz;
+    }
+    const SweepShape &sh = b->sweep;
+    const int64_t slots =
+        int64_t(b->cu_count) * std::max(1, 4 * sh.waves * 64 / (sh.tx * sh.ty));
+    int best = 1;
+    int64_t best_cost = -1;
+    for (int nz = 1; nz <= 64; ++nz) {
+        int64_t tiles = 0;
+        for (int m = 0; m < b->n; ++m) {
+            if (all || !b->dropped[m]) {
+                const int en = b->f[m].nx + 1;
+                tiles += int64_t((en + sh.tx - 2) / (sh.tx - 1)) *
+                         ((en + sh.ty - 2) / (sh.ty - 1)) * ((en + nz - 1) / nz);
+            }
+        }
+        const int64_t cost = (tiles + slots - 1) / slots * (nz + 3);
+        if (best_cost < 0 || cost <= best_cost) {
+            best_cost = cost;
+            best = nz;
+        }
+    }
+    return best;
+}
+
 // tiles of the sweep (for the current shape) and element chunks of the
 // members still in the lists
 void cut_work(lulesh_batch *b, bool all)
 {
     b->tiles.clear();
     b->chunks.clear();
+    if (b->plan) {
+        b->sweep.nz = plan_planes(b, all);
+    }
     const int tx = b->sweep.tx, ty = b->sweep.ty, nz = b->sweep.nz;
     for (int m = 0; m < b->n; ++m) {
         if (!all && b->dropped[m]) {
@@ -171,7 +229,33 @@ void cut_work(lulesh_batch *b, bool all)
             b->chunks.push_back(make_int2(m, c * kChunk));
         }
     }
+    // in XCD order (xcd_order): neighbouring tiles share an L2
+    std::vector<int4> t;
+    t.reserve(b->tiles.size());
+    const size_t per = (b->tiles.size() + 7) / 8;
+    for (size_t r = 0; r < per; ++r) {
+        for (size_t x = 0; x < 8; ++x) {
+            if (x * per + r < b->tiles.size()) t.push_back(b->tiles[x * per + r]);
+        }
+    }
+    b->tiles.swap(t);
     order_eos_chunks(b, all);
+}
+
+// room for n entries in a device list that is about to be written
+template <typename T>
+int make_room(lulesh_batch *b, T **list, size_t *room, size_t n)
+{
+    if (n <= *room) {
+        return LULESH_OK;
+    }
+    BHIP_TRY(b, hipStreamSynchronize(b->stream));
+    if (*list) (void)hipFree(*list);
+    *list = nullptr;
+    *room = 0;
+    BHIP_TRY(b, hipMalloc(list, n * sizeof(T)));
+    *room = n;
+    return LULESH_OK;
 }
 
 // uploads the work lists (and their counts) for the members not dropped;
@@ -183,7 +267,13 @@ int upload_work(lulesh_batch *b)
     w.num_members = b->n;
     w.num_tiles = int(b->tiles.size());
     w.num_chunks = int(b->chunks.size());
+    w.num_eos = int(b->eos_chunks.size());
+    w.planes = b->sweep.nz;
+    w.eos_elems = b->eos_elems;
     w.num_pending = 0;
+    int rc = make_room(b, &b->d_tiles, &b->tiles_room, b->tiles.size());
+    if (rc) return rc;
+    if ((rc = make_room(b, &b->d_eos_chunks, &b->eos_room, b->eos_chunks.size()))) return rc;
     w.tiles = b->d_tiles;
     w.chunks = b->d_chunks;
     w.eos_chunks = b->d_eos_chunks;
@@ -206,7 +296,8 @@ int upload_work(lulesh_batch *b)
     return LULESH_OK;
 }
 
-// the full list sizes fix the grids of the captured launches
+// The grids of the captured launches: the full lists', and as many blocks as
+// the lists of fewer members are cut into.
 void size_grids(lulesh_batch *b)
 {
     cut_work(b, true);
@@ -216,7 +307,15 @@ void size_grids(lulesh_batch *b)
 
 int sweep_grid(const lulesh_batch *b)
 {
-    return b->sweep_blocks > 0 ? std::min(b->sweep_blocks, b->full_tiles) : b->full_tiles;
+    if (b->sweep_blocks > 0) {
+        return std::min(b->sweep_blocks, b->full_tiles);
+    }
+    return b->plan ? std::max(b->full_tiles, 8 * b->cu_count) : b->full_tiles;
+}
+
+int eos_grid(const lulesh_batch *b)
+{
+    return std::max(b->full_chunks, int(kEosSmallBlocks) + b->n);
 }
 
 int elem_grid(const lulesh_batch *b)
@@ -246,7 +345,8 @@ int queue_cycles(lulesh_batch *b, int ncycles)
                                dim3(ge), dim3(kChunk), 0, st, b->d_members, b->d_work,
                                b->prm);
             BHIP_TRY(b, hipGetLastError());
-            hipLaunchKernelGGL(fz ? fused::k_q_eos_dt_chunks : k_q_eos_dt_chunks, dim3(ge),
+            hipLaunchKernelGGL(fz ? fused::k_q_eos_dt_chunks : k_q_eos_dt_chunks,
+                               dim3(eos_grid(b)),
                                dim3(kChunk), 0, st, b->d_members, b->d_work, b->prm);
         } else {
             hipLaunchKernelGGL(fz ? fused::k_kinematics_q_batch : k_kinematics_q_batch,
@@ -401,14 +501,14 @@ int batch_build(lulesh_batch *b, const lulesh_config *cfg, const double *efactor
     std::vector<BatchMember> members(size_t(b->n));
     std::vector<DevScalars> scalars(size_t(b->n));
     b->f.resize(size_t(b->n));
-    b->eos_passes.resize(size_t(b->n));
+    b->eos_extra.resize(size_t(b->n));
     for (int m = 0; m < b->n; ++m) {
         DevScalars *unused = nullptr;  // the members' scalars live contiguously
         carve_domain(static_cast<char *>(b->arena) + offset[m], meshes[m], b->f[m],
                      &unused);
         BHIP_TRY(b, upload_mesh(meshes[m], b->f[m], b->stream));
         members[m].f = b->f[m];
-        b->eos_passes[size_t(m)] = eos_block_passes(meshes[m].elem_rep);
+        b->eos_extra[size_t(m)] = eos_block_extra(meshes[m].elem_rep, kEosBlockLeast);
         members[m].s = b->d_scalars + m;
         scalars[m] = initial_scalars(meshes[m], cfg[m].stoptime, cfg[m].max_cycles);
     }
@@ -420,14 +520,9 @@ int batch_build(lulesh_batch *b, const lulesh_config *cfg, const double *efactor
                                hipMemcpyHostToDevice, b->stream));
     BHIP_TRY(b, hipStreamSynchronize(b->stream));
 
-    // work lists: room for the largest cut of any supported shape is not
-    // known in advance, so size for the finest one (16 x 4 tiles, nz = 1)
-    // lazily in set_shape; here for the default shape
     b->dropped.assign(size_t(b->n), 0);
     size_grids(b);
-    BHIP_TRY(b, hipMalloc(&b->d_tiles, size_t(std::max(b->full_tiles, 1)) * sizeof(int4)));
     BHIP_TRY(b, hipMalloc(&b->d_chunks, size_t(std::max(b->full_chunks, 1)) * sizeof(int2)));
-    BHIP_TRY(b, hipMalloc(&b->d_eos_chunks, size_t(std::max(b->full_chunks, 1)) * sizeof(int2)));
     return upload_work(b);
 }
 
@@ -636,21 +731,16 @@ int lulesh_batch_set_shape(lulesh_batch *b, int tx, int ty, int nz, int waves,
     if (!force_sweep_shape_supported(sh)) {
         return bfail(b, LULESH_BAD_ARG, "sweep shape not built into the library");
     }
-    const bool recut = sh.tx != b->sweep.tx || sh.ty != b->sweep.ty || sh.nz != b->sweep.nz;
+    const bool recut = b->plan || sh.tx != b->sweep.tx || sh.ty != b->sweep.ty ||
+                       sh.nz != b->sweep.nz;
     b->sweep = sh;
+    b->plan = false;
     b->sweep_blocks = sweep_blocks;
     b->elem_blocks = elem_blocks;
     b->cycles_per_graph = cycles_per_graph;
     drop_graph(b);
     if (recut) {
-        const int old_tiles = b->full_tiles;
         size_grids(b);
-        if (b->full_tiles > old_tiles) {
-            BHIP_TRY(b, hipStreamSynchronize(b->stream));
-            BHIP_TRY(b, hipFree(b->d_tiles));
-            b->d_tiles = nullptr;
-            BHIP_TRY(b, hipMalloc(&b->d_tiles, size_t(b->full_tiles) * sizeof(int4)));
-        }
         return upload_work(b);
     }
     return LULESH_OK;

@@ -765,9 +765,9 @@ __global__ __launch_bounds__(TX *TY, W) void k_force_sweep(DevFields f, DevScala
 // leave their tiles at once (sweep_tile reads their flags).
 template <int TX, int TY, int W>
 __global__ __launch_bounds__(TX *TY, W) void k_force_sweep_batch(
-    const BatchMember *__restrict__ members, const BatchWork *__restrict__ work, PhysParams prm, int nz)
+    const BatchMember *__restrict__ members, const BatchWork *__restrict__ work, PhysParams prm)
 {
-    const int n = work->num_tiles;
+    const int n = work->num_tiles, nz = work->planes;
     const LULESH_AS_GLOBAL int32_t *tiles = (const LULESH_AS_GLOBAL int32_t *)work->tiles;
     for (int t = int(blockIdx.x); t < n; t += int(gridDim.x)) {
         __syncthreads();  // the LDS of the previous tile is no longer read
@@ -789,12 +789,12 @@ hipError_t launch_shape(int nz, const DevFields &f, DevScalars *s,
 }
 
 template <int TX, int TY, int W>
-hipError_t launch_shape_batch(int nz, int blocks, const BatchMember *members,
+hipError_t launch_shape_batch(int blocks, const BatchMember *members,
                               const BatchWork *work, const PhysParams &prm,
                               hipStream_t stream)
 {
     hipLaunchKernelGGL((k_force_sweep_batch<TX, TY, W>), dim3(blocks), dim3(TX * TY), 0,
-                       stream, members, work, prm, nz);
+                       stream, members, work, prm);
     return hipGetLastError();
 }
 
@@ -1241,12 +1241,12 @@ hipError_t launch_force_sweep_batch(const SweepShape &sh, int blocks,
                                     const BatchMember *members, const BatchWork *work,
                                     const PhysParams &prm, hipStream_t stream)
 {
-    if (sh.nz < 1 || blocks < 1) {
+    if (blocks < 1) {
         return hipErrorInvalidValue;
     }
 #define LULESH_LAUNCH(a, b, w)                                                  \
     if (sh.tx == a && sh.ty == b && sh.waves == w)                              \
-        return launch_shape_batch<a, b, w>(sh.nz, blocks, members, work, prm, stream);
+        return launch_shape_batch<a, b, w>(blocks, members, work, prm, stream);
     LULESH_SWEEP_SHAPES(LULESH_LAUNCH)
 #undef LULESH_LAUNCH
     return hipErrorInvalidValue;

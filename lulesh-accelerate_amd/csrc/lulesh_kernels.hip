@@ -1276,7 +1276,7 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_batch(const BatchMember *__res
     __shared__ unsigned long long lds_c[4], lds_h[4];
     __shared__ int skip;
     __shared__ RepLds rep_lds;
-    const int n = work->num_chunks;
+    const int n = work->num_eos;
     const LULESH_AS_GLOBAL int32_t *chunks = (const LULESH_AS_GLOBAL int32_t *)work->eos_chunks;
     for (int c = int(blockIdx.x); c < n; c += int(gridDim.x)) {
         const BatchMember &m = members[chunks[2 * c]];
@@ -1290,8 +1290,8 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_batch(const BatchMember *__res
         }
         __builtin_amdgcn_s_setprio(1);  // the element's loads first
         const int el = chunks[2 * c + 1] + int(threadIdx.x);
-        q_eos_dt_nat_block(global_view(m.f), m.s, prm, el, el < m.f.num_elem, lds_c, lds_h,
-                           rep_lds);
+        const bool valid = int(threadIdx.x) < work->eos_elems && el < m.f.num_elem;
+        q_eos_dt_nat_block(global_view(m.f), m.s, prm, el, valid, lds_c, lds_h, rep_lds);
     }
 }
 
@@ -1303,7 +1303,7 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_chunks(const BatchMember *__re
     __shared__ int skip;
     __shared__ RepLds rep_lds;
     const int c = int(blockIdx.x);
-    if (c >= work->num_chunks) {
+    if (c >= work->num_eos) {
         return;
     }
     const LULESH_AS_GLOBAL int32_t *chunks = (const LULESH_AS_GLOBAL int32_t *)work->eos_chunks;
@@ -1317,7 +1317,8 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_chunks(const BatchMember *__re
     }
     __builtin_amdgcn_s_setprio(1);  // the element's loads first
     const int el = chunks[2 * c + 1] + int(threadIdx.x);
-    q_eos_dt_nat_block(global_view(m.f), m.s, prm, el, el < m.f.num_elem, lds_c, lds_h, rep_lds);
+    const bool valid = int(threadIdx.x) < work->eos_elems && el < m.f.num_elem;
+    q_eos_dt_nat_block(global_view(m.f), m.s, prm, el, valid, lds_c, lds_h, rep_lds);
 }
 
 // ---------------------------------------------------------------------------

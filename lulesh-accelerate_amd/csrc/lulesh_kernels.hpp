@@ -436,10 +436,13 @@ struct BatchWork {
     int num_members;
     int num_tiles;    // force-sweep tiles (member, bx, by, bz)
     int num_chunks;   // element chunks (member, first element)
+    int num_eos;      // Q/EOS chunks, of eos_elems elements
+    int planes;       // node planes per tile
+    int eos_elems;
     int num_pending;  // members with cycles left, set by k_dt_finish_batch
     int4 *tiles;
     int2 *chunks;      // in mesh order, for the kinematics
-    int2 *eos_chunks;  // the same chunks in the Q/EOS dispatch order
+    int2 *eos_chunks;  // in the Q/EOS dispatch order
 };
 
 __global__ void k_time_increment(DevScalars *s, int ic_mode);

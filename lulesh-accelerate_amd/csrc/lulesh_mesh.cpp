@@ -324,10 +324,8 @@ HostMesh build_mesh(const MeshConfig &cfg)
 // everywhere there is nothing to share (45^3 44.8, 43.9, 43.8).
 int eos_block_elems(int64_t num_elem, bool repeated)
 {
-    constexpr int kLeast = 64;
-    constexpr int64_t kMostBlocks = 2700;
     int elems = kEosBlockElems;
-    while (repeated && elems > kLeast && num_elem <= kMostBlocks * (elems / 2)) {
+    while (repeated && elems > kEosBlockLeast && num_elem <= kEosSmallBlocks * (elems / 2)) {
         elems /= 2;
     }
     return elems;
@@ -339,17 +337,23 @@ constexpr double kHeavyCost = 1.0, kHeavySpan = 0.75;
 
 }  // namespace
 
-std::vector<int64_t> eos_block_passes(const std::vector<uint16_t> &rep, int elems)
+std::vector<int32_t> eos_block_extra(const std::vector<uint16_t> &rep, int elems)
 {
     const size_t ne = rep.size(), be = size_t(elems);
-    const size_t g = (ne + be - 1) / be;
-    std::vector<int64_t> passes(g);
-    for (size_t b = 0; b < g; ++b) {
-        int64_t extra = 0;
+    std::vector<int32_t> extra((ne + be - 1) / be, 0);
+    for (size_t b = 0; b < extra.size(); ++b) {
         for (size_t i = b * be; i < std::min(ne, (b + 1) * be); ++i) {
-            extra += int64_t(rep[i]) - 1;
+            extra[b] += int32_t(rep[i]) - 1;
         }
-        passes[b] = 1 + (extra + kEosBlockElems - 1) / kEosBlockElems;
+    }
+    return extra;
+}
+
+std::vector<int64_t> eos_block_passes(const std::vector<uint16_t> &rep, int elems)
+{
+    std::vector<int64_t> passes;
+    for (int32_t extra : eos_block_extra(rep, elems)) {
+        passes.push_back(1 + (int64_t(extra) + kEosBlockElems - 1) / kEosBlockElems);
     }
     return passes;
 }

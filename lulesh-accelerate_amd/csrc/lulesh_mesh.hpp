@@ -48,8 +48,11 @@ struct HostMesh {
 // Threads, and elements at most, of a block of the mesh-order Q/EOS kernels.
 constexpr int kEosBlockElems = 256;
 
-// The elements of such a block in the launch of one domain, fewer than its
-// threads where the domain is small and has repetitions to share.
+// The elements of such a block, fewer than its threads where the launch has
+// few elements and repetitions to share: kEosBlockLeast at least, and not so
+// few that the blocks exceed kEosSmallBlocks.
+constexpr int kEosBlockLeast = 64;
+constexpr int64_t kEosSmallBlocks = 2700;
 int eos_block_elems(int64_t num_elem, bool repeated);
 
 // The order in which the blocks of a mesh-order Q/EOS launch take the mesh's
@@ -57,10 +60,12 @@ int eos_block_elems(int64_t num_elem, bool repeated);
 // lulesh_mesh.cpp): slot t of the launch processes block order[t].
 std::vector<int32_t> eos_block_order(const std::vector<uint16_t> &rep,
                                      int elems = kEosBlockElems);
-// Its two parts: the EOS passes of each block (one, plus the evaluations
+// Its parts: the evaluations beyond each element's first of each block, the
+// EOS passes of each block (one, plus the evaluations
 // beyond each element's first shared over the block), and the launch order
 // of blocks of the given costs, listed in the order whose locality the
 // launch should keep.
+std::vector<int32_t> eos_block_extra(const std::vector<uint16_t> &rep, int elems);
 std::vector<int64_t> eos_block_passes(const std::vector<uint16_t> &rep,
                                       int elems = kEosBlockElems);
 std::vector<int32_t> spread_costly_blocks(const std::vector<int64_t> &passes);

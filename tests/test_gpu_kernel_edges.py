@@ -135,3 +135,22 @@ def test_state_there_and_back(lulesh_gpu, oracle, nx, mode):
         d.set(f, st[f][::-1].copy())
         assert np.array_equal(d.get(f), st[f][::-1])
     d.close()
+
+
+# 75^3 beside the others: chunks of 256 elements; without it 64.  Planes per
+# tile follow the members left, to the last one alone.
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("sizes", [[75, 30, 5], [31, 12, 44, 1, 16]])
+def test_ensemble_cut_anew_as_members_stop(lulesh_gpu, sizes, fused):
+    """Members of a default ensemble against runs of their own, bit for bit."""
+    b = lulesh_gpu.Batch(sizes, fused=fused)
+    b.run()
+    for m, nx in enumerate(sizes):
+        d = lulesh_gpu.Domain(nx, fused=fused)
+        rc, cycles = d.run()
+        assert b.stats(m)[0] == rc and b.stats(m)[1].cycle == cycles
+        bad = [f for f in NODE + ELEM[:10] if not np.array_equal(
+            b.get(m, f).view(np.uint64), d.get(f).view(np.uint64))]
+        assert bad == []
+        d.close()
+    b.close()
