@@ -249,10 +249,12 @@ int launch(lulesh_domain *d, int kid, F &&body)
 
 int queue_cycle_u(lulesh_domain *d)
 {
-    const unsigned ge = unsigned((d->num_elem + kBlock - 1) / kBlock);
+    // whole rounds over the XCDs (xcd_order)
+    auto grid8 = [](int64_t blocks) { return unsigned((blocks + 7) / 8 * 8); };
+    const unsigned ge = grid8((d->num_elem + kBlock - 1) / kBlock);
     const DevForceBlocksU &b = d->fblocks;  // a renumbered mesh
     // k_nodes_u: eight lanes per boundary node (num_boundary <= 2^27)
-    const unsigned gb = unsigned((8 * int64_t(b.num_boundary) + kBlock - 1) / kBlock);
+    const unsigned gb = grid8((8 * int64_t(b.num_boundary) + kBlock - 1) / kBlock);
     hipStream_t st = d->stream;
     DevScalars *s = d->s;
     const DevFields &f = d->f;
@@ -266,7 +268,7 @@ int queue_cycle_u(lulesh_domain *d)
         return rc;
     if (b.num_blocks > 0 && (rc = launch(d, KID_FORCES_U, [&] {
              hipLaunchKernelGGL(fused ? fused::k_forces_u_blocks : k_forces_u_blocks,
-                                dim3(unsigned(b.num_blocks)), dim3(kForceBlockElems), 0, st,
+                                dim3(grid8(b.num_blocks)), dim3(kForceBlockElems), 0, st,
                                 f, m, b, s, p);
          })))
         return rc;

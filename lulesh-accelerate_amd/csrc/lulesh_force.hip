@@ -995,6 +995,163 @@ constexpr bool kOneSlot = true;
 constexpr bool kOneSlot = false;
 #endif
 
+#ifdef LULESH_FUSED
+// As the bit-identical build's kernel below, with an element's stress and
+// hourglass forces formed together in its modes (lulesh_modal.hpp): 624
+// instead of 1033 FP64 instructions a thread, one staging in LDS and two
+// barriers instead of four.  100^3 as a mesh 139 -> 109 us, 61^3 34.5 -> 27.6.
+// One block fits on a CU, so its loads (about 340 MB in all at 100^3, 3.1
+// TB/s) and its arithmetic take turns.  Two blocks of 128 VGPRs, the loads in
+// six dependent steps and one component staged at a time, took 140 us (with
+// spills 160 to 234); one block per CU looping, the next block's lists
+// fetched ahead, 114.  Blocks in XCD order: 119 -> 111 us (bit-identical 179
+// -> 172).
+__global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields f, DevMeshU m,
+                                                                      DevForceBlocksU b,
+                                                                      DevScalars *s,
+                                                                      PhysParams prm)
+{
+    constexpr int kN = kForceBlockElems;
+    __shared__ double corner[3][8][kN];
+    __shared__ int skip, s_par;
+    __shared__ double s_dt;
+    const int blk = xcd_order(int(blockIdx.x), b.num_blocks), l = int(threadIdx.x);
+    if (blk >= b.num_blocks) {
+        return;  // the whole block
+    }
+    // other blocks may raise an error meanwhile: read the flags once per
+    // block, so that every thread takes the same path to the barriers
+    if (threadIdx.x == 0) {
+        skip = (s->active == 0 || s->error != 0) ? 1 : 0;
+        s_par = s->cur;
+        s_dt = s->deltatime;
+    }
+    const int ne = f.num_elem;
+    const int el = b.elem_start[blk] + l;
+    const bool has = el < b.elem_start[blk + 1];
+    const int node = b.node_start[blk] + l;
+    const bool own = node < b.node_start[blk + 1];
+    const unsigned e = unsigned(has ? el : 0);
+    unsigned nodes[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        nodes[c] = unsigned(load_at(m.nodelist, unsigned(c * ne) + e));
+    }
+    int slot[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        slot[c] = load_at(m.corner_slot, unsigned(c * ne) + e);
+    }
+    int cb = 0, ce = 0;
+    if (own) {
+        cb = b.ncorner_start[node];
+        ce = b.ncorner_start[node + 1];
+    }
+    __syncthreads();
+    if (skip) {
+        return;
+    }
+    const int par = wave_uniform(s_par);
+    const double dt = wave_uniform(s_dt);
+    double xyz[3][8], vel[3][8];
+    const double *const pos[3] = {parity_copy(f.x, par), parity_copy(f.y, par),
+                                  parity_copy(f.z, par)};
+    const double *const dot[3] = {parity_copy(f.xd, par), parity_copy(f.yd, par),
+                                  parity_copy(f.zd, par)};
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            xyz[t][c] = load_at(pos[t], nodes[c]);
+        }
+    }
+    const double vol = load_at(f.v, e);
+    const double determ = load_at(f.volo, e) * vol;
+    const double press = load_at(f.p, e) + load_at(f.q, e);
+    const double ssm = load_at(f.ss, e) * load_at(f.elem_mass, e);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            vel[t][c] = load_at(dot[t], nodes[c]);
+        }
+    }
+    NodeU nd{1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0};
+    int corners[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        corners[i] = cb + i < ce ? int(b.ncorners[cb + i]) : -1;
+    }
+    if (own) {
+        nd = load_node_u(f, m, par, node);
+    }
+    {
+        const double hgc = prm.hgcoef > 0.0 ? -prm.hgcoef * 0.01 : 0.0;
+        const double coef = hg_over_root(hgc * ssm, hg_root(determ));
+        ForceShape<double> sh;
+        force_shape(corner_modes(xyz[0]), corner_modes(xyz[1]), corner_modes(xyz[2]),
+                    elem_recip(determ), sh);
+        // VolumeError on the Jacobian volume, then on v, which the
+        // reference tests for every element before it looks at hgcoef
+        // (:1579-1584, :1540-1543)
+        if (has && (sh.det <= 0.0 || vol <= 0.0)) {
+            atomicCAS(&s->error, 0, -1);
+        }
+        double v[3][8];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const double n1 = t == 0 ? sh.n[0].x : t == 1 ? sh.n[0].y : sh.n[0].z;
+            const double n2 = t == 0 ? sh.n[1].x : t == 1 ? sh.n[1].y : sh.n[1].z;
+            const double n3 = t == 0 ? sh.n[2].x : t == 1 ? sh.n[2].y : sh.n[2].z;
+            const ElemModes<double> F = force_modes(sh, n1, n2, n3, press * 0.015625, coef,
+                                                    corner_modes(vel[t]));
+            // the corners' values from the modes, by faces, low and high
+            const double face[2][4] = {{-F.a3, F.a1 - F.h2, F.a2 - F.h1, F.h3 - F.h4},
+                                       {F.a3, F.a1 + F.h2, F.a2 + F.h1, F.h3 + F.h4}};
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const double ap = face[h][0] + face[h][1], am = face[h][0] - face[h][1];
+                const double bp = face[h][2] + face[h][3], bm = face[h][2] - face[h][3];
+                v[t][4 * h] = am - bm;
+                v[t][4 * h + 1] = ap - bp;
+                v[t][4 * h + 2] = ap + bp;
+                v[t][4 * h + 3] = am + bm;
+            }
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                corner[t][c][l] = v[t][c];
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            if (has && slot[c] >= 0) {
+                store_corner(m.bs, slot[c], v[0][c], v[1][c], v[2][c]);
+            }
+        }
+    }
+    __syncthreads();
+    double sum[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        if (corners[i] >= 0) {
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                sum[t] += corner[t][corners[i] & 7][corners[i] >> 3];
+            }
+        }
+    }
+    for (int i = cb + 8; i < ce; ++i) {
+        const int k = b.ncorners[i];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            sum[t] += corner[t][k & 7][k >> 3];
+        }
+    }
+    if (own) {
+        move_node_u(f, par, dt, prm, node, nd, sum[0], sum[1], sum[2]);
+    }
+}
+#else
 // One block of elements (b.elem_start[blockIdx.x] ..., consecutive), one
 // element per thread, then the block's interior nodes (consecutive), one per
 // thread.  The stress corners and then the hourglass corners are staged in
@@ -1022,7 +1179,10 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
     if (skip) {
         return;
     }
-    const int blk = int(blockIdx.x), l = int(threadIdx.x);
+    const int blk = xcd_order(int(blockIdx.x), b.num_blocks), l = int(threadIdx.x);
+    if (blk >= b.num_blocks) {
+        return;  // the whole block
+    }
     const int ne = f.num_elem;
     const int par = s->cur;
     const double dt = s->deltatime;
@@ -1062,7 +1222,7 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
             for (int t = 0; t < 3; ++t) {
                 corner[t][c][l] = fs[t][c];
             }
-            if (slot[c] >= 0 && (!kOneSlot || !hourglass)) {
+            if (slot[c] >= 0) {
                 store_corner(m.bs, slot[c], fs[0][c], fs[1][c], fs[2][c]);
             }
         }
@@ -1082,16 +1242,11 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
             hourglass_corners_u(E, prm, fh);
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
-                if (kOneSlot && slot[c] >= 0) {
-                    // the element's own stress corner, still in LDS
-                    store_corner(m.bs, slot[c], corner[0][c][l] + fh[0][c],
-                                 corner[1][c][l] + fh[1][c], corner[2][c][l] + fh[2][c]);
-                }
 #pragma unroll
                 for (int t = 0; t < 3; ++t) {
                     corner[t][c][l] = fh[t][c];
                 }
-                if (!kOneSlot && slot[c] >= 0) {
+                if (slot[c] >= 0) {
                     store_corner(m.bh, slot[c], fh[0][c], fh[1][c], fh[2][c]);
                 }
             }
@@ -1113,6 +1268,8 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
     }
 }
 
+#endif
+
 // The boundary nodes first .. first + count - 1, eight lanes per node:
 // gather of their corners from their slots, acceleration, symmetry planes,
 // velocity and position (:905-926, :1475-1496, :1613-1683), in place (the
@@ -1129,7 +1286,7 @@ __global__ __launch_bounds__(256) void k_nodes_u(DevFields f, DevMeshU m, DevSca
     if (s->active == 0 || s->error != 0) {
         return;
     }
-    const int t = int(blockIdx.x) * int(blockDim.x) + int(threadIdx.x);
+    const int t = xcd_order(int(blockIdx.x), int(gridDim.x)) * int(blockDim.x) + int(threadIdx.x);
     const int i = t / kLanes, q = t % kLanes, l = int(threadIdx.x);
     // a group lies in one wave and leaves whole: its lanes share i
     if (i >= count) {

@@ -315,6 +315,10 @@ __device__ __forceinline__ double load_at(const LULESH_AS_GLOBAL double *p, unsi
 {
     return *(const LULESH_AS_GLOBAL double *)((const LULESH_AS_GLOBAL char *)p + idx * 8u);
 }
+__device__ __forceinline__ int32_t load_at(const int32_t *p, unsigned idx)
+{
+    return *reinterpret_cast<const int32_t *>(reinterpret_cast<const char *>(p) + idx * 4u);
+}
 __device__ __forceinline__ void store_at(double *p, unsigned idx, double v)
 {
     *reinterpret_cast<double *>(reinterpret_cast<char *>(p) + idx * 8u) = v;

@@ -154,3 +154,22 @@ def test_ensemble_cut_anew_as_members_stop(lulesh_gpu, sizes, fused):
         assert bad == []
         d.close()
     b.close()
+
+
+# element blocks of at most 512: one, one and a bit, and several on each XCD
+@pytest.mark.parametrize("nx,cycles", [(1, 8), (2, 20), (8, 20), (9, 20), (17, 40), (33, 20)])
+@pytest.mark.parametrize("fused", [False, True])
+def test_mesh_forces_by_blocks(lulesh_gpu, oracle, nx, cycles, fused):
+    """A cube given as lists against the cube itself with the same initial
+    conditions: the same bits, fused within the reference's tolerance."""
+    a = lulesh_gpu.Domain.from_mesh(oracle.cube_mesh(nx), fused=fused)
+    b = lulesh_gpu.Domain(nx, ic_mode=1)
+    assert a.step(cycles) == b.step(cycles)
+    for f in NODE + ELEM[:11]:
+        x, y = a.get(f), b.get(f)
+        if fused:
+            assert np.max(np.abs(x - y)) <= 1e-10 * np.max(np.abs(y)), f
+        else:
+            assert np.array_equal(x.view(np.uint64), y.view(np.uint64)), f
+    a.close()
+    b.close()
