@@ -55,6 +55,7 @@ constexpr int kBatch = 32;  // cycles queued per host round trip in run()
 // cycles per captured graph: lulesh_step replays a graph of this many cycles
 // as often as it fits and queues the rest one launch at a time
 constexpr int kGraphCycles = 32;
+static_assert(kGraphCycles % 2 == 0, "a graph ends on the copy of the scalars it began with");
 
 // Planes (or layers) per block of a sweep that cuts `planes` of them into
 // chunks, `cols` blocks each, `resident` of which a CU holds.  A block takes
@@ -151,7 +152,7 @@ struct lulesh_domain {
     int learned_form = 0;               // LULESH_LEARNED_FACTORS / _STANDIN
     DevFields f{};
     DevFieldsMixed fm{};
-    DevScalars *s = nullptr;
+    DevScalars *s = nullptr;  // two copies (start_cycle); between calls the first holds
     PhysParams prm{};
     SweepShape sweep = kDefaultSweep;
     bool limit_sweep = false;  // the fused kinematics and limiter in one sweep
@@ -247,7 +248,7 @@ int launch(lulesh_domain *d, int kid, F &&body)
     return LULESH_OK;
 }
 
-int queue_cycle_u(lulesh_domain *d)
+int queue_cycle_u(lulesh_domain *d, const DevScalars *from, DevScalars *s)
 {
     // whole rounds over the XCDs (xcd_order)
     auto grid8 = [](int64_t blocks) { return unsigned((blocks + 7) / 8 * 8); };
@@ -256,20 +257,15 @@ int queue_cycle_u(lulesh_domain *d)
     // k_nodes_u: eight lanes per boundary node (num_boundary <= 2^27)
     const unsigned gb = grid8((8 * int64_t(b.num_boundary) + kBlock - 1) / kBlock);
     hipStream_t st = d->stream;
-    DevScalars *s = d->s;
     const DevFields &f = d->f;
     const DevMeshU &m = d->mesh;
     const PhysParams &p = d->prm;
     const bool fused = d->fused;
     int rc;
-    if ((rc = launch(d, KID_TIME_INCREMENT, [&] {
-             hipLaunchKernelGGL(k_time_increment, dim3(1), dim3(64), 0, st, s, p.ic_mode);
-         })))
-        return rc;
     if (b.num_blocks > 0 && (rc = launch(d, KID_FORCES_U, [&] {
              hipLaunchKernelGGL(fused ? fused::k_forces_u_blocks : k_forces_u_blocks,
                                 dim3(grid8(b.num_blocks)), dim3(kForceBlockElems), 0, st,
-                                f, m, b, s, p);
+                                f, m, b, from, s, p);
          })))
         return rc;
     if (gb > 0 && (rc = launch(d, KID_NODES_U, [&] {
@@ -291,16 +287,18 @@ int queue_cycle_u(lulesh_domain *d)
     return LULESH_OK;
 }
 
-// store: whether the fused cycle leaves the intermediate fields (delv, the Q
-// gradients) in memory: the last cycle of a call does
-int queue_cycle(lulesh_domain *d, bool store)
+// Cycle c of a call (start_cycle says what c decides).  store: whether the
+// fused cycle leaves the intermediate fields (delv, the Q gradients) in
+// memory: the last cycle of a call does.
+int queue_cycle(lulesh_domain *d, int c, bool store)
 {
+    const DevScalars *const from = d->s + (c & 1);
+    DevScalars *const s = d->s + (~c & 1);
     if (d->unstructured) {
-        return queue_cycle_u(d);
+        return queue_cycle_u(d, from, s);
     }
     const unsigned ge = unsigned((d->num_elem + kBlock - 1) / kBlock);
     hipStream_t st = d->stream;
-    DevScalars *s = d->s;
     const DevFields &f = d->f;
     const DevFieldsMixed &fm = d->fm;
     const int eos_elems = d->mixed ? fm.eos_elems : f.eos_elems;
@@ -308,17 +306,13 @@ int queue_cycle(lulesh_domain *d, bool store)
     const PhysParams &p = d->prm;
     const bool mixed = d->mixed;
     int rc;
-    if ((rc = launch(d, KID_TIME_INCREMENT, [&] {
-             hipLaunchKernelGGL(k_time_increment, dim3(1), dim3(64), 0, st, s, p.ic_mode);
-         })))
-        return rc;
     const bool fused = d->fused;
     if ((rc = launch(d, KID_FORCE_SWEEP, [&]() -> hipError_t {
              if (mixed) {
-                 return launch_force_sweep_mixed(d->sweep, fm, s, p, st);
+                 return launch_force_sweep_mixed(d->sweep, fm, from, s, p, st);
              }
-             return fused ? fused::launch_force_sweep(d->sweep, f, s, p, st)
-                          : launch_force_sweep(d->sweep, f, s, p, st);
+             return fused ? fused::launch_force_sweep(d->sweep, f, from, s, p, st)
+                          : launch_force_sweep(d->sweep, f, from, s, p, st);
          })))
         return rc;
     // unless another Q phase is set (the learned closure, the region-sorted
@@ -416,7 +410,7 @@ int ensure_graph(lulesh_domain *d)
     HIP_TRY(d, hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
     int rc = LULESH_OK;
     for (int c = 0; c < kGraphCycles && rc == LULESH_OK; ++c) {
-        rc = queue_cycle(d, c + 1 == kGraphCycles);
+        rc = queue_cycle(d, c, c + 1 == kGraphCycles);
     }
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(d->stream, &g);
@@ -451,8 +445,8 @@ int read_scalars(lulesh_domain *d, DevScalars *out)
 
 int write_scalars(lulesh_domain *d, const DevScalars &in)
 {
-    HIP_TRY(d, hipMemcpyAsync(d->s, &in, sizeof(DevScalars), hipMemcpyHostToDevice,
-                              d->stream));
+    const DevScalars both[2] = {in, in};
+    HIP_TRY(d, hipMemcpyAsync(d->s, both, sizeof(both), hipMemcpyHostToDevice, d->stream));
     HIP_TRY(d, hipStreamSynchronize(d->stream));
     return LULESH_OK;
 }
@@ -724,8 +718,8 @@ int build_device_domain_u(lulesh_domain *d, const HostMeshU &m, const ForceBlock
         b.ncorners = u16;
     }
     DevScalars *sc = nullptr;
-    const std::vector<DevScalars> one(1);
-    if ((rc = upload_vec(d, one, &sc))) return rc;
+    const std::vector<DevScalars> two(2);
+    if ((rc = upload_vec(d, two, &sc))) return rc;
     d->s = sc;
     HIP_TRY(d, hipStreamSynchronize(d->stream));
     HostMesh hm;  // the loop scalars of the 1.0 ICs
@@ -929,13 +923,13 @@ int lulesh_step(lulesh_domain *d, int ncycles, int *cycles_done)
         }
     }
     for (; c < ncycles; ++c) {
-        if ((rc = queue_cycle(d, c + 1 == ncycles))) return rc;
+        if ((rc = queue_cycle(d, c, c + 1 == ncycles))) return rc;
     }
     // the last cycle's time constraints (the others were applied by the
     // following cycle's TimeIncrement)
     if ((rc = launch(d, KID_DT_FINISH, [&] {
-             hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(64), 0, d->stream, d->s,
-                                d->prm.ic_mode);
+             hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(64), 0, d->stream,
+                                d->s + (ncycles & 1), d->s, d->prm.ic_mode);
          })))
         return rc;
     HIP_TRY(d, hipEventRecord(d->step_end, d->stream));

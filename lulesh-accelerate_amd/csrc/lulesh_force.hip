@@ -71,8 +71,8 @@ constexpr int kStencil[8][6] = {{1, 2, 3, 4, 5, 7}, {2, 3, 0, 5, 6, 4},
 //    spill).
 //  - The LDS this frees holds the next plane and the next layer's corners
 //    beside the current ones: one barrier per layer (two: 157 us).
-template <int TX, int TY, class Fields>
-__device__ __forceinline__ void sweep_tile(const Fields &f, DevScalars *s,
+template <int TX, int TY, bool Starts, class Fields>
+__device__ __forceinline__ void sweep_tile(const Fields &f, const DevScalars *from, DevScalars *s,
                                            const PhysParams &prm, int nz, int bx,
                                            int by, int bz)
 {
@@ -89,10 +89,16 @@ __device__ __forceinline__ void sweep_tile(const Fields &f, DevScalars *s,
 
     const int tid = threadIdx.x;
     if (tid == 0) {
-        // the flags are only changed by earlier kernels: read them once
-        s_go = (s->active != 0 && s->error == 0) ? 1 : 0;
-        s_par = s->cur;
-        s_dt = s->deltatime;
+        CycleStart c;
+        if constexpr (Starts) {
+            c = start_cycle(from, s, prm.ic_mode, bx == 0 && by == 0 && bz == 0);
+        } else {
+            // the flags are only changed by earlier kernels: read them once
+            c = {(s->active != 0 && s->error == 0) ? 1 : 0, s->cur, s->deltatime};
+        }
+        s_go = c.go;
+        s_par = c.par;
+        s_dt = c.dt;
     }
     __syncthreads();
     if (!s_go) {
@@ -351,8 +357,8 @@ __device__ __forceinline__ void sweep_tile(const Fields &f, DevScalars *s,
 // moving loads up, so a load issued in the layer that uses it waits for
 // HBM), and the owned node is copied to registers so that the next node
 // plane is stored inside the layer's last fold: four barriers per layer.
-template <int TX, int TY, class Fields>
-__device__ __forceinline__ void sweep_tile(const Fields &f, DevScalars *s,
+template <int TX, int TY, bool Starts, class Fields>
+__device__ __forceinline__ void sweep_tile(const Fields &f, const DevScalars *from, DevScalars *s,
                                            const PhysParams &prm, int nz, int bx,
                                            int by, int bz)
 {
@@ -366,10 +372,16 @@ __device__ __forceinline__ void sweep_tile(const Fields &f, DevScalars *s,
 
     const int tid = threadIdx.x;
     if (tid == 0) {
-        // the flags are only changed by earlier kernels: read them once
-        s_go = (s->active != 0 && s->error == 0) ? 1 : 0;
-        s_par = s->cur;
-        s_dt = s->deltatime;
+        CycleStart c;
+        if constexpr (Starts) {
+            c = start_cycle(from, s, prm.ic_mode, bx == 0 && by == 0 && bz == 0);
+        } else {
+            // the flags are only changed by earlier kernels: read them once
+            c = {(s->active != 0 && s->error == 0) ? 1 : 0, s->cur, s->deltatime};
+        }
+        s_go = c.go;
+        s_par = c.par;
+        s_dt = c.dt;
     }
     __syncthreads();
     if (!s_go) {
@@ -746,8 +758,9 @@ __device__ __forceinline__ void sweep_tile(const Fields &f, DevScalars *s,
 // from 895 to 580 MB in both builds, and the fused build from 165 to 157 us;
 // the exact build, bounded by FP64 issue, stays at 290.
 template <int TX, int TY, int W>
-__global__ __launch_bounds__(TX *TY, W) void k_force_sweep(DevFields f, DevScalars *s,
-                                                        PhysParams prm, int nz)
+__global__ __launch_bounds__(TX *TY, W) void k_force_sweep(DevFields f,
+                                                        const DevScalars *__restrict__ from,
+                                                        DevScalars *s, PhysParams prm, int nz)
 {
     const int nbx = (f.nx + TX - 1) / (TX - 1), nby = (f.nx + TY - 1) / (TY - 1);
     const int tiles = nbx * nby * ((f.nx + nz) / nz);
@@ -756,7 +769,7 @@ __global__ __launch_bounds__(TX *TY, W) void k_force_sweep(DevFields f, DevScala
         return;
     }
     const int r = t / nbx, bz = r / nby;
-    sweep_tile<TX, TY>(f, s, prm, nz, t - r * nbx, r - bz * nby, bz);
+    sweep_tile<TX, TY, true>(f, from, s, prm, nz, t - r * nbx, r - bz * nby, bz);
 }
 
 // The ensemble form: a grid walks the tile list of all members (one block
@@ -772,19 +785,19 @@ __global__ __launch_bounds__(TX *TY, W) void k_force_sweep_batch(
     for (int t = int(blockIdx.x); t < n; t += int(gridDim.x)) {
         __syncthreads();  // the LDS of the previous tile is no longer read
         const BatchMember &m = members[tiles[4 * t]];
-        sweep_tile<TX, TY>(global_view(m.f), m.s, prm, nz, tiles[4 * t + 1],
+        sweep_tile<TX, TY, false>(global_view(m.f), nullptr, m.s, prm, nz, tiles[4 * t + 1],
                                   tiles[4 * t + 2], tiles[4 * t + 3]);
     }
 }
 
 template <int TX, int TY, int W>
-hipError_t launch_shape(int nz, const DevFields &f, DevScalars *s,
+hipError_t launch_shape(int nz, const DevFields &f, const DevScalars *from, DevScalars *s,
                         const PhysParams &prm, hipStream_t stream)
 {
     const int64_t tiles = int64_t((f.nx + TX - 1) / (TX - 1)) *
                           ((f.nx + TY - 1) / (TY - 1)) * ((f.nx + nz) / nz);
-    hipLaunchKernelGGL((k_force_sweep<TX, TY, W>), dim3(unsigned((tiles + 7) / 8 * 8)), dim3(TX * TY), 0, stream, f,
-                       s, prm, nz);
+    hipLaunchKernelGGL((k_force_sweep<TX, TY, W>), dim3(unsigned((tiles + 7) / 8 * 8)),
+                       dim3(TX * TY), 0, stream, f, from, s, prm, nz);
     return hipGetLastError();
 }
 
@@ -1008,23 +1021,19 @@ constexpr bool kOneSlot = false;
 // -> 172).
 __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields f, DevMeshU m,
                                                                       DevForceBlocksU b,
+                                                                      const DevScalars *from,
                                                                       DevScalars *s,
                                                                       PhysParams prm)
 {
     constexpr int kN = kForceBlockElems;
     __shared__ double corner[3][8][kN];
-    __shared__ int skip, s_par;
-    __shared__ double s_dt;
+    __shared__ CycleStart start;
     const int blk = xcd_order(int(blockIdx.x), b.num_blocks), l = int(threadIdx.x);
     if (blk >= b.num_blocks) {
         return;  // the whole block
     }
-    // other blocks may raise an error meanwhile: read the flags once per
-    // block, so that every thread takes the same path to the barriers
-    if (threadIdx.x == 0) {
-        skip = (s->active == 0 || s->error != 0) ? 1 : 0;
-        s_par = s->cur;
-        s_dt = s->deltatime;
+    if (l == 0) {
+        start = start_cycle(from, s, prm.ic_mode, blk == 0);
     }
     const int ne = f.num_elem;
     const int el = b.elem_start[blk] + l;
@@ -1048,11 +1057,11 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
         ce = b.ncorner_start[node + 1];
     }
     __syncthreads();
-    if (skip) {
+    if (!start.go) {
         return;
     }
-    const int par = wave_uniform(s_par);
-    const double dt = wave_uniform(s_dt);
+    const int par = wave_uniform(start.par);
+    const double dt = wave_uniform(start.dt);
     double xyz[3][8], vel[3][8];
     const double *const pos[3] = {parity_copy(f.x, par), parity_copy(f.y, par),
                                   parity_copy(f.z, par)};
@@ -1164,28 +1173,27 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
 // blocks still compute.
 __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields f, DevMeshU m,
                                                                       DevForceBlocksU b,
+                                                                      const DevScalars *from,
                                                                       DevScalars *s,
                                                                       PhysParams prm)
 {
     constexpr int kN = kForceBlockElems;
     __shared__ double corner[3][8][kN];
-    __shared__ int skip;
-    // other blocks may raise an error meanwhile: read the flags once per
-    // block, so that every thread takes the same path to the barriers
-    if (threadIdx.x == 0) {
-        skip = (s->active == 0 || s->error != 0) ? 1 : 0;
-    }
-    __syncthreads();
-    if (skip) {
-        return;
-    }
+    __shared__ CycleStart start;
     const int blk = xcd_order(int(blockIdx.x), b.num_blocks), l = int(threadIdx.x);
     if (blk >= b.num_blocks) {
         return;  // the whole block
     }
+    if (l == 0) {
+        start = start_cycle(from, s, prm.ic_mode, blk == 0);
+    }
+    __syncthreads();
+    if (!start.go) {
+        return;
+    }
     const int ne = f.num_elem;
-    const int par = s->cur;
-    const double dt = s->deltatime;
+    const int par = start.par;
+    const double dt = start.dt;
     const int e0 = b.elem_start[blk];
     const int el = e0 + l;
     const bool has = el < b.elem_start[blk + 1];
@@ -1380,15 +1388,15 @@ bool force_sweep_shape_supported(const SweepShape &sh)
 }
 
 hipError_t launch_force_sweep(const SweepShape &sh, const DevFields &f,
-                              DevScalars *s, const PhysParams &prm,
-                              hipStream_t stream)
+                              const DevScalars *from, DevScalars *s,
+                              const PhysParams &prm, hipStream_t stream)
 {
     if (sh.nz < 1) {
         return hipErrorInvalidValue;
     }
 #define LULESH_LAUNCH(a, b, w)                            \
     if (sh.tx == a && sh.ty == b && sh.waves == w)        \
-        return launch_shape<a, b, w>(sh.nz, f, s, prm, stream);
+        return launch_shape<a, b, w>(sh.nz, f, from, s, prm, stream);
     LULESH_SWEEP_SHAPES(LULESH_LAUNCH)
 #undef LULESH_LAUNCH
     return hipErrorInvalidValue;

@@ -3,8 +3,8 @@
 // Cycle = TimeIncrement + LagrangeLeapFrog (reference/C/LULESH-OMP.cc:
 // 3179-3188; lulesh-2.0.3/lulesh.cc:2771-2781).  Kernels, in launch order:
 //
-//   k_time_increment   TimeIncrement, on the device (:557-604)
-//   k_force_sweep      LagrangeNodal: forces, acceleration, boundary
+//   k_force_sweep      TimeIncrement (:557-604; start_cycle), then
+//                      LagrangeNodal: forces, acceleration, boundary
 //                      conditions, velocity, position (lulesh_force.hip)
 //   k_kinematics_q     per element: kinematics and the monotonic-Q gradients
 //                      (:1927-2180)
@@ -73,28 +73,6 @@ __device__ __forceinline__ void raise_error(DevScalars *s, int code)
     atomicCAS(&s->error, 0, code);
 }
 
-// The Courant and hydro minima of a cycle are gathered in the accumulators
-// by k_q_eos_dt and applied here, at the next kernel boundary: by the next
-// cycle's TimeIncrement or by the k_dt_finish that closes a batch.
-__device__ __forceinline__ void apply_constraints(DevScalars *s, int ic_mode)
-{
-    if (!s->dt_pending) {
-        return;
-    }
-    s->dt_pending = 0;
-    if (s->error != 0) {
-        return;
-    }
-    const double c = from_bits(s->acc_courant);
-    const double h = from_bits(s->acc_hydro);
-    if (ic_mode == 2) {
-        s->dtcourant = kBig;
-        s->dthydro = kBig;
-    }
-    if (c < kBig) s->dtcourant = c;
-    if (h < kBig) s->dthydro = h;
-}
-
 // a + b of two products, each rounded on its own
 __device__ __forceinline__ double add(double a, double b)
 {
@@ -116,73 +94,6 @@ __device__ __forceinline__ void elem_ijk(const F &f, int el, int &i, int &j,
 
 }  // namespace
 
-// ---------------------------------------------------------------------------
-// TimeIncrement (reference/C/LULESH-OMP.cc:557-604; lulesh-2.0.3/lulesh.cc:
-// 194-251).  Decides whether this cycle runs at all: the loop condition of
-// the drivers (time < stoptime, and cycle < its for 2.0) is evaluated here.
-// ---------------------------------------------------------------------------
-namespace {
-
-__device__ __forceinline__ void time_increment(DevScalars *s, int ic_mode)
-{
-    apply_constraints(s, ic_mode);
-    if (s->error != 0 || !(s->time < s->stoptime) || !(s->cycle < s->max_cycles)) {
-        s->active = 0;
-        return;
-    }
-    s->active = 1;
-    double targetdt = s->stoptime - s->time;
-    if ((s->dtfixed <= 0.0) && (s->cycle != 0)) {
-        double ratio;
-        const double olddt = s->deltatime;
-        double newdt = kBig;
-        if (s->dtcourant < newdt) {
-            newdt = s->dtcourant / 2.0;
-        }
-        if (s->dthydro < newdt) {
-            newdt = s->dthydro * 2.0 / 3.0;
-        }
-        ratio = newdt / olddt;
-        if (ratio >= 1.0) {
-            if (ratio < s->deltatimemultlb) {
-                newdt = olddt;
-            } else if (ratio > s->deltatimemultub) {
-                newdt = olddt * s->deltatimemultub;
-            }
-        }
-        if (newdt > s->dtmax) {
-            newdt = s->dtmax;
-        }
-        s->deltatime = newdt;
-    }
-    if ((targetdt > s->deltatime) && (targetdt < (4.0 * s->deltatime / 3.0))) {
-        targetdt = 2.0 * s->deltatime / 3.0;
-    }
-    if (targetdt < s->deltatime) {
-        s->deltatime = targetdt;
-    }
-    s->time += s->deltatime;
-    ++s->cycle;
-    s->cur ^= 1;  // this cycle's nodes go to the other copy
-    s->last = (!(s->time < s->stoptime) || !(s->cycle < s->max_cycles)) ? 1 : 0;
-    s->acc_courant = as_bits(kBig);
-    s->acc_hydro = as_bits(kBig);
-    s->dt_pending = 1;
-}
-
-}  // namespace
-
-__global__ void k_time_increment(DevScalars *s, int ic_mode)
-{
-    if (threadIdx.x == 0) {
-        // on a copy in registers: one batch of loads and one of stores, not a
-        // wait for memory at every field the pointer form might alias
-        DevScalars t = *s;
-        time_increment(&t, ic_mode);
-        *s = t;
-    }
-}
-
 // one thread per member
 __global__ void k_time_increment_batch(const BatchMember *__restrict__ members,
                                        const BatchWork *__restrict__ work, int ic_mode)
@@ -190,7 +101,7 @@ __global__ void k_time_increment_batch(const BatchMember *__restrict__ members,
     const int n = work->num_members;
     for (int m = int(threadIdx.x); m < n; m += int(blockDim.x)) {
         DevScalars *const s = members[m].s;
-        DevScalars t = *s;  // on a register copy, as in k_time_increment
+        DevScalars t = *s;  // on a register copy, as in start_cycle
         time_increment(&t, ic_mode);
         *s = t;
     }
@@ -1558,10 +1469,12 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_u(DevFields f, DevMeshU m, Dev
 // applies the minima of the last cycle: 2.0 starts every cycle from 1e20
 // (lulesh-2.0.3/lulesh.cc:2616-2620); 1.0 keeps the previous constraint when
 // no element gave one (reference/C/LULESH-OMP.cc:2867-2871)
-__global__ void k_dt_finish(DevScalars *s, int ic_mode)
+__global__ void k_dt_finish(const DevScalars *from, DevScalars *s, int ic_mode)
 {
     if (threadIdx.x == 0) {
-        apply_constraints(s, ic_mode);
+        DevScalars t = *from;
+        apply_constraints(&t, ic_mode);
+        *s = t;
     }
 }
 

@@ -70,7 +70,8 @@ __device__ __forceinline__ void elem_ijk(const DevFieldsMixed &f, int el, int &i
 // (lulesh_force.hip), with float32 corner forces.
 // ---------------------------------------------------------------------------
 template <int TX, int TY>
-__device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f, DevScalars *s,
+__device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
+                                                 const DevScalars *from, DevScalars *s,
                                                  const PhysParams &prm, int nz, int bx,
                                                  int by, int bz)
 {
@@ -84,9 +85,11 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f, DevSca
 
     const int tid = threadIdx.x;
     if (tid == 0) {
-        s_go = (s->active != 0 && s->error == 0) ? 1 : 0;
-        s_par = s->cur;
-        s_dt = s->deltatime;
+        const CycleStart c =
+            start_cycle(from, s, prm.ic_mode, bx == 0 && by == 0 && bz == 0);
+        s_go = c.go;
+        s_par = c.par;
+        s_dt = c.dt;
     }
     __syncthreads();
     if (!s_go) {
@@ -416,6 +419,7 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f, DevSca
 // tiles in the order of k_force_sweep, whose reason holds here too
 template <int TX, int TY, int W>
 __global__ __launch_bounds__(TX *TY, W) void k_force_sweep_mixed(DevFieldsMixed f,
+                                                              const DevScalars *__restrict__ from,
                                                               DevScalars *s,
                                                               PhysParams prm, int nz)
 {
@@ -426,17 +430,17 @@ __global__ __launch_bounds__(TX *TY, W) void k_force_sweep_mixed(DevFieldsMixed 
         return;
     }
     const int r = t / nbx, bz = r / nby;
-    sweep_tile_mixed<TX, TY>(f, s, prm, nz, t - r * nbx, r - bz * nby, bz);
+    sweep_tile_mixed<TX, TY>(f, from, s, prm, nz, t - r * nbx, r - bz * nby, bz);
 }
 
 template <int TX, int TY, int W>
-hipError_t launch_mixed_shape(int nz, const DevFieldsMixed &f, DevScalars *s,
-                              const PhysParams &prm, hipStream_t stream)
+hipError_t launch_mixed_shape(int nz, const DevFieldsMixed &f, const DevScalars *from,
+                              DevScalars *s, const PhysParams &prm, hipStream_t stream)
 {
     const int64_t tiles = int64_t((f.nx + TX - 1) / (TX - 1)) *
                           ((f.nx + TY - 1) / (TY - 1)) * ((f.nx + nz) / nz);
     hipLaunchKernelGGL((k_force_sweep_mixed<TX, TY, W>), dim3(unsigned((tiles + 7) / 8 * 8)),
-                       dim3(TX * TY), 0, stream, f, s, prm, nz);
+                       dim3(TX * TY), 0, stream, f, from, s, prm, nz);
     return hipGetLastError();
 }
 
@@ -1021,15 +1025,15 @@ bool force_sweep_mixed_shape_supported(const SweepShape &sh)
 }
 
 hipError_t launch_force_sweep_mixed(const SweepShape &sh, const DevFieldsMixed &f,
-                                    DevScalars *s, const PhysParams &prm,
-                                    hipStream_t stream)
+                                    const DevScalars *from, DevScalars *s,
+                                    const PhysParams &prm, hipStream_t stream)
 {
     if (sh.nz < 1) {
         return hipErrorInvalidValue;
     }
 #define LULESH_LAUNCH(a, b, w)                     \
     if (sh.tx == a && sh.ty == b && sh.waves == w) \
-        return launch_mixed_shape<a, b, w>(sh.nz, f, s, prm, stream);
+        return launch_mixed_shape<a, b, w>(sh.nz, f, from, s, prm, stream);
     LULESH_MIXED_SHAPES(LULESH_LAUNCH)
 #undef LULESH_LAUNCH
     return hipErrorInvalidValue;

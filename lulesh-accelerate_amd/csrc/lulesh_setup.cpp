@@ -54,7 +54,7 @@ size_t domain_arena_bytes(const HostMesh &m)
     size_t bytes = (kNodeArrays * pn + kElemArrays * pe) * sizeof(double);
     bytes += round_up(pe * sizeof(int32_t), 256) + 2 * round_up(pe * sizeof(uint16_t), 256);
     bytes += round_up(m.eos_launch.size() * sizeof(int32_t), 256);
-    bytes += round_up(sizeof(DevScalars), 256);
+    bytes += round_up(2 * sizeof(DevScalars), 256);
     return bytes;
 }
 
@@ -157,7 +157,7 @@ size_t domain_arena_bytes_mixed(const HostMesh &m)
                    kElemArrays32 * pe * sizeof(float);
     bytes += round_up(pe * sizeof(int32_t), 256) + 2 * round_up(pe * sizeof(uint16_t), 256);
     bytes += round_up(m.eos_launch.size() * sizeof(int32_t), 256);
-    bytes += round_up(sizeof(DevScalars), 256);
+    bytes += round_up(2 * sizeof(DevScalars), 256);
     return bytes;
 }
 
