@@ -57,6 +57,18 @@ constexpr int kBatch = 32;  // cycles queued per host round trip in run()
 constexpr int kGraphCycles = 32;
 static_assert(kGraphCycles % 2 == 0, "a graph ends on the copy of the scalars it began with");
 
+int compute_units()
+{
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
+            hipSuccess ||
+        cus < 1) {
+        cus = 256;
+    }
+    return cus;
+}
+
 // Planes (or layers) per block of a sweep that cuts `planes` of them into
 // chunks, `cols` blocks each, `resident` of which a CU holds.  A block takes
 // its planes one after another, so a launch lasts as many rounds of the
@@ -75,14 +87,7 @@ static_assert(kGraphCycles % 2 == 0, "a graph ends on the copy of the scalars it
 int plan_planes(int planes, long long cols, int resident, int extra)
 {
     constexpr int most = 64;
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
-            hipSuccess ||
-        cus < 1) {
-        cus = 256;
-    }
-    const long long slots = (long long)resident * cus;
+    const long long slots = (long long)resident * compute_units();
     int best = 1;
     long long best_cost = -1;
     for (int nz = 1; nz <= std::min(planes, most); ++nz) {
@@ -155,6 +160,7 @@ struct lulesh_domain {
     DevScalars *s = nullptr;  // two copies (start_cycle); between calls the first holds
     PhysParams prm{};
     SweepShape sweep = kDefaultSweep;
+    bool plane_blocks = false;  // launch_force_planes in place of the bit-identical sweep
     bool limit_sweep = false;  // the fused kinematics and limiter in one sweep
     int limit_planes = 1;      //   and its element layers per block
     void *arena = nullptr;
@@ -311,6 +317,9 @@ int queue_cycle(lulesh_domain *d, int c, bool store)
              if (mixed) {
                  return launch_force_sweep_mixed(d->sweep, fm, from, s, p, st);
              }
+             if (!fused && d->plane_blocks) {
+                 return launch_force_planes(f, from, s, p, st);
+             }
              return fused ? fused::launch_force_sweep(d->sweep, f, from, s, p, st)
                           : launch_force_sweep(d->sweep, f, from, s, p, st);
          })))
@@ -382,6 +391,7 @@ std::vector<unsigned char> launch_signature(const lulesh_domain *d)
     put(&d->s, sizeof(d->s));
     put(&d->prm, sizeof(d->prm));
     put(&d->sweep, sizeof(d->sweep));
+    put(&d->plane_blocks, sizeof(d->plane_blocks));
     put(&d->limit_sweep, sizeof(d->limit_sweep));
     put(&d->limit_planes, sizeof(d->limit_planes));
     put(&d->mesh, sizeof(d->mesh));
@@ -545,6 +555,8 @@ int create_domain(const lulesh_config *cfg, bool mixed, double efactor,
     if (cfg->nx >= 1 && cfg->nx <= 600) {
         const int64_t nx = cfg->nx;
         d->sweep.nz = default_sweep_planes(d->sweep, cfg->nx, mixed);
+        // two blocks on a CU, all in one round
+        d->plane_blocks = !mixed && force_planes_blocks(cfg->nx) <= 2 * compute_units();
         d->limit_sweep = limiter_in_sweep(nx * nx * nx, (nx + 1) * (nx + 1) * (nx + 1));
         d->limit_planes = plan_planes(cfg->nx, fused::kinematics_limit_columns(cfg->nx), 3, 5);
     }
@@ -1154,6 +1166,7 @@ int lulesh_set_sweep_shape(lulesh_domain *d, int tx, int ty, int nz, int waves)
         return fail(d, LULESH_BAD_ARG, "sweep shape not built into the library");
     }
     d->sweep = sh;
+    d->plane_blocks = false;  // the caller's shape is a sweep's
     return LULESH_OK;
 }
 

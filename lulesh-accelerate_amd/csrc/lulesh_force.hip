@@ -25,6 +25,8 @@
 // LDS (one global read per node per block) and the advanced nodes are
 // written to the other copy.
 #include "lulesh_kernels.hpp"
+
+#include <type_traits>
 #include "lulesh_mesh.hpp"
 
 #include "lulesh_elem.hpp"
@@ -1363,6 +1365,190 @@ __global__ __launch_bounds__(256) void k_nodes_u(DevFields f, DevMeshU m, DevSca
         move_node_u(f, par, dt, prm, n, nd, fx, fy, fz);
     }
 }
+
+#ifndef LULESH_FUSED
+// The sweep of a small domain: one block per tile and node plane, which
+// forms the element layers below and above the plane side by side, 128
+// threads each, where a sweep block takes them one after another.  With at
+// most two blocks per CU, in one round, the launch lasts as long as a block,
+// whose FP64 instructions wait for each other: two waves per SIMD overlap,
+// one does not.  The element arithmetic and every sum's order are the
+// sweep's, so the bits are.
+// Kernel between events (6 us of them the events), against the sweep with one
+// plane per block: 10^3 10.4 against 16.8 us, 30^3 13.5 against 17.6, 33^3
+// 14.3 against 33.9; 15^3 and 16^3 16 against 17.  Tiles of 32 x 4 need more
+// than one round from 31^3 (33 us); 8 x 8: 30^3 17.7 us.
+namespace {
+
+constexpr int kPlaneTX = 16, kPlaneTY = 8;
+
+template <int TX, int TY>
+__global__ __launch_bounds__(2 * TX *TY, 2) void k_force_planes(DevFields f,
+                                                                const DevScalars *__restrict__ from,
+                                                                DevScalars *s, PhysParams prm)
+{
+    constexpr int NT = TX * TY, PX = TX + 1, PN = (TX + 1) * (TY + 1);
+    __shared__ double plane[3][6][PN];            // node planes k - 1, k, k + 1
+    __shared__ double corner[2][2][3][4][NT];     // stress, hourglass; of the lower layer its
+                                                  // corners 4 .. 7, of the upper 0 .. 3
+    __shared__ double hsum[3][NT];
+    __shared__ CycleStart start;
+    const int nx = f.nx, en = nx + 1;
+    const int nbx = (nx + TX - 1) / (TX - 1), nby = (nx + TY - 1) / (TY - 1);
+    const int t = xcd_order(int(blockIdx.x), nbx * nby * en);
+    if (t >= nbx * nby * en) {
+        return;
+    }
+    const int row = t / nbx, bx = t - row * nbx, k = row / nby, by = row - k * nby;
+    if (threadIdx.x == 0) {
+        start = start_cycle(from, s, prm.ic_mode, t == 0);
+    }
+    const int g = wave_uniform(int(threadIdx.x) / NT);  // 0: the layer below, 1: above
+    const int tid = int(threadIdx.x) % NT;
+    const int tx = tid % TX, ty = tid / TX;
+    const int ie = bx * (TX - 1) - 1 + tx, je = by * (TY - 1) - 1 + ty, ke = k - 1 + g;
+    const bool has = ie >= 0 && ie < nx && je >= 0 && je < nx && ke >= 0 && ke < nx;
+    const bool own = tx >= 1 && ty >= 1 && ie <= nx && je <= nx;
+    ElemU E;
+    if (has) {
+        const unsigned e = unsigned((ke * nx + je) * nx + ie);
+        E.p = load_at(f.p, e);
+        E.q = load_at(f.q, e);
+        E.v = load_at(f.v, e);
+        E.volo = load_at(f.volo, e);
+        E.ss = load_at(f.ss, e);
+        E.emass = load_at(f.elem_mass, e);
+    }
+    const int node = (k * en + je) * en + ie;
+    const double mass = own ? f.nodal_mass[node] : 1.0;
+    __syncthreads();
+    if (!start.go) {
+        return;
+    }
+    const int par = wave_uniform(start.par);
+    const double dt = wave_uniform(start.dt);
+    // nodes outside the domain stand for their nearest: only elements that
+    // are none read them
+    constexpr int kSlots = (3 * PN + 2 * NT - 1) / (2 * NT);
+#pragma unroll
+    for (int r = 0; r < kSlots; ++r) {
+        const int i = int(threadIdx.x) + r * 2 * NT;
+        if (i < 3 * PN) {
+            const int p = i / PN, q = i - p * PN;
+            const int gi = min(max(bx * (TX - 1) - 1 + q % PX, 0), nx);
+            const int gj = min(max(by * (TY - 1) - 1 + q / PX, 0), nx);
+            const int gk = min(max(k - 1 + p, 0), nx);
+            const unsigned n = unsigned((gk * en + gj) * en + gi);
+            const double *const in[6] = {f.x[par ^ 1],  f.y[par ^ 1],  f.z[par ^ 1],
+                                         f.xd[par ^ 1], f.yd[par ^ 1], f.zd[par ^ 1]};
+#pragma unroll
+            for (int fld = 0; fld < 6; ++fld) {
+                plane[p][fld][q] = load_at(in[fld], n);
+            }
+        }
+    }
+    __syncthreads();
+    const bool hourglass = prm.hgcoef > 0.0;
+    const int base = ty * PX + tx;
+    const int off[4] = {base, base + 1, base + PX + 1, base + PX};
+    // C0: the first of the layer's corners in this plane
+    auto forces = [&](auto layer) {
+        constexpr int G = decltype(layer)::value, C0 = G == 0 ? 4 : 0;
+        double c8[3][8] = {};
+        if (has) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const double(&pl)[6][PN] = plane[G + c / 4];
+                const int o = off[c % 4];
+                E.x[c] = pl[0][o];
+                E.y[c] = pl[1][o];
+                E.z[c] = pl[2][o];
+                E.vel[0][c] = pl[3][o];
+                E.vel[1][c] = pl[4][o];
+                E.vel[2][c] = pl[5][o];
+            }
+            if (stress_corners_u(E, c8)) {
+                atomicCAS(&s->error, 0, -1);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                corner[0][G][t][c][tid] = c8[t][C0 + c];
+            }
+        }
+        if (hourglass) {
+            if (has) {
+                hourglass_corners_u(E, prm, c8);
+            }
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    corner[1][G][t][c][tid] = c8[t][C0 + c];
+                }
+            }
+        }
+    };
+    if (g == 0) {
+        forces(std::integral_constant<int, 0>());
+    } else {
+        forces(std::integral_constant<int, 1>());
+    }
+    __syncthreads();
+    // the lower half adds the stress corners of its nodes, the upper half the
+    // hourglass corners: 6, 7, 5, 4 of the layer below, 2, 3, 1, 0 of the
+    // layer above, as the sweep's fold
+    double F[3] = {0.0, 0.0, 0.0};
+    if (own && (g == 0 || hourglass)) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+#pragma unroll
+            for (int layer = 0; layer < 2; ++layer) {
+                const double(&c)[4][NT] = corner[g][layer][t];
+                F[t] += c[2][tid - TX - 1];
+                F[t] += c[3][tid - TX];
+                F[t] += c[1][tid - 1];
+                F[t] += c[0][tid];
+            }
+            if (g == 1) {
+                hsum[t][tid] = F[t];
+            }
+        }
+    }
+    __syncthreads();
+    if (own && g == 0) {
+        if (hourglass) {
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                F[t] += hsum[t][tid];
+            }
+        }
+        const int sym = (ie == 0 ? 1 : 0) | (je == 0 ? 2 : 0) | (k == 0 ? 4 : 0);
+        const NodeU nd{mass,           plane[1][0][base], plane[1][1][base], plane[1][2][base],
+                       plane[1][3][base], plane[1][4][base], plane[1][5][base], sym};
+        move_node_u(f, par, dt, prm, node, nd, F[0], F[1], F[2]);
+    }
+}
+
+}  // namespace
+
+int force_planes_blocks(int nx)
+{
+    return ((nx + kPlaneTX - 1) / (kPlaneTX - 1)) * ((nx + kPlaneTY - 1) / (kPlaneTY - 1)) *
+           (nx + 1);
+}
+
+hipError_t launch_force_planes(const DevFields &f, const DevScalars *from, DevScalars *s,
+                               const PhysParams &prm, hipStream_t stream)
+{
+    const unsigned blocks = unsigned((force_planes_blocks(f.nx) + 7) / 8 * 8);
+    hipLaunchKernelGGL((k_force_planes<kPlaneTX, kPlaneTY>), dim3(blocks),
+                       dim3(2 * kPlaneTX * kPlaneTY), 0, stream, f, from, s, prm);
+    return hipGetLastError();
+}
+#endif
 
 // (TX, TY, minimum waves per SIMD the register budget must allow); the
 // number of node planes per block is a launch argument

@@ -596,6 +596,11 @@ __global__ void k_dt_finish_batch(const BatchMember *members, BatchWork *work,
 hipError_t launch_force_sweep(const SweepShape &shape, const DevFields &f,
                               const DevScalars *from, DevScalars *s,
                               const PhysParams &prm, hipStream_t stream);
+// The same of a small domain, a block per node plane (bit-identical build), and
+// its number of blocks.
+hipError_t launch_force_planes(const DevFields &f, const DevScalars *from, DevScalars *s,
+                               const PhysParams &prm, hipStream_t stream);
+int force_planes_blocks(int nx);
 // The ensemble sweep: `blocks` persistent blocks over work->tiles, which
 // must have been cut for the same shape (tx, ty, nz).
 hipError_t launch_force_sweep_batch(const SweepShape &shape, int blocks,

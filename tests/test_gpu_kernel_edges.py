@@ -173,3 +173,27 @@ def test_mesh_forces_by_blocks(lulesh_gpu, oracle, nx, cycles, fused):
             assert np.array_equal(x.view(np.uint64), y.view(np.uint64)), f
     a.close()
     b.close()
+
+
+# tiles of 16 x 8 columns own 15 x 7 nodes: one tile, its edge, several; 33^3
+# the largest in one round, 34^3 swept
+@pytest.mark.parametrize("nx,mode,hgcoef", [(1, 2, None), (2, 1, None), (6, 2, None),
+                                            (7, 2, 0.0), (14, 2, None), (15, 1, None),
+                                            (16, 2, None), (30, 2, None), (33, 2, None),
+                                            (33, 1, 0.0), (34, 2, None)])
+def test_plane_blocks_are_the_sweep(lulesh_gpu, nx, mode, hgcoef):
+    """The forces of a small domain by blocks of one node plane, bit for bit
+    the sweep's, with and without hourglass forces."""
+    a = lulesh_gpu.Domain(nx, ic_mode=mode)
+    b = lulesh_gpu.Domain(nx, ic_mode=mode)
+    b.set_sweep_shape(32, 8, 4, 2)
+    if hgcoef is not None:
+        a.set_parameter("hgcoef", hgcoef)
+        b.set_parameter("hgcoef", hgcoef)
+    ra, rb = a.step(37, raise_on_error=False), b.step(37, raise_on_error=False)
+    assert ra == rb
+    bad = [f for f in NODE + ELEM
+           if not np.array_equal(a.get(f).view(np.uint64), b.get(f).view(np.uint64))]
+    assert bad == []
+    a.close()
+    b.close()
