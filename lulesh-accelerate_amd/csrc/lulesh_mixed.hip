@@ -22,6 +22,7 @@
 #include "lulesh_kernels.hpp"
 
 #include "lulesh_elem.hpp"
+#include "lulesh_modal.hpp"
 
 #pragma clang fp contract(fast)
 
@@ -30,11 +31,6 @@ namespace lulesh {
 namespace {
 
 constexpr double kBig = 1.0e+20;
-
-constexpr int kStencil[8][6] = {{1, 2, 3, 4, 5, 7}, {2, 3, 0, 5, 6, 4},
-                                {3, 0, 1, 6, 7, 5}, {0, 1, 2, 7, 4, 6},
-                                {7, 6, 5, 0, 3, 1}, {4, 7, 6, 1, 0, 2},
-                                {5, 4, 7, 2, 1, 3}, {6, 5, 4, 3, 2, 0}};
 
 __device__ __forceinline__ float frcp(float v) { return __builtin_amdgcn_rcpf(v); }
 __device__ __forceinline__ float frsq(float v) { return __builtin_amdgcn_rsqf(v); }
@@ -66,8 +62,18 @@ __device__ __forceinline__ void elem_ijk(const DevFieldsMixed &f, int el, int &i
 }
 
 // ---------------------------------------------------------------------------
-// Force sweep: the tiling, staging and node order of sweep_tile
-// (lulesh_force.hip), with float32 corner forces.
+// Force sweep: the tiling of sweep_tile (lulesh_force.hip), with an element's
+// stress and hourglass forces formed together in its modes
+// (lulesh_modal.hpp), in float32, and a node's eight corners summed in
+// float64.
+//
+// Against the two kinds corner by corner, staged one after the other and
+// summed in float32: 120^3 step 193 -> 174 us, 150^3 373 -> 341, 91^3 97 -> 87
+// (per thread and layer 1187 instead of 1629 vector instructions, two
+// barriers instead of four in the staging).  Error against the float64 run
+// over nine domains of 20^3 to 200^3, 100 to 900 cycles: the run's time 0.79
+// and p 1.01 of what it was, in the geometric mean; summed in float32, 1.2 to
+// 1.3.
 // ---------------------------------------------------------------------------
 template <int TX, int TY>
 __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
@@ -111,7 +117,6 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
     const int je = j0 - 1 + ty;
     const bool col_valid = ie >= 0 && ie < nx && je >= 0 && je < nx;
     const bool owner = tx >= 1 && ty >= 1 && ie <= nx && je <= nx;
-    const bool hourglass = prm.hgcoef > 0.0;
     // corner slots of element columns outside the domain hold +0.0, so the
     // fold adds four corners per layer without testing which elements exist
     // (adding +0.0 to a sum started from +0.0 changes no bits)
@@ -124,7 +129,7 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
             }
         }
     }
-    const float hg = float(-prm.hgcoef * 0.01);
+    const float hg = prm.hgcoef > 0.0 ? float(-prm.hgcoef * 0.01) : 0.0f;
 
     constexpr int kSlots = (PN + NT - 1) / NT;
     int gnode[kSlots];
@@ -171,29 +176,29 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
         }
     };
     // wave priority rises as a barrier approaches, as in the float64 sweep:
-    // 2 in the folds, the nodal update and the plane store, 1 in the stress
-    // arithmetic and the hourglass projection, 0 in the volume derivatives
-    auto fold = [&](bool finalize, bool carry, bool layer, float *F, float *P) {
+    // 2 in the folds, the nodal update and the plane store, 1 in the element
+    // arithmetic
+    auto fold = [&](bool finalize, bool carry, bool layer, double *F, double *P) {
         __syncthreads();
         __builtin_amdgcn_s_setprio(2);
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
             if (finalize) {
-                float acc = P[t];
+                double acc = P[t];
                 if (layer) {
-                    acc += corner[t][2][tid - TX - 1];
-                    acc += corner[t][3][tid - TX];
-                    acc += corner[t][1][tid - 1];
-                    acc += corner[t][0][tid];
+                    acc += double(corner[t][2][tid - TX - 1]);
+                    acc += double(corner[t][3][tid - TX]);
+                    acc += double(corner[t][1][tid - 1]);
+                    acc += double(corner[t][0][tid]);
                 }
                 F[t] = acc;
             }
             if (carry) {
-                float acc = 0.0f;
-                acc += corner[t][6][tid - TX - 1];
-                acc += corner[t][7][tid - TX];
-                acc += corner[t][5][tid - 1];
-                acc += corner[t][4][tid];
+                double acc = 0.0;
+                acc += double(corner[t][6][tid - TX - 1]);
+                acc += double(corner[t][7][tid - TX]);
+                acc += double(corner[t][5][tid - 1]);
+                acc += double(corner[t][4][tid]);
                 P[t] = acc;
             }
         }
@@ -203,7 +208,7 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
     const int base = ty * PX + tx;
     const int nodeoff[4] = {base, base + 1, base + PX + 1, base + PX};
 
-    float P[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    double P[3] = {0.0, 0.0, 0.0};
     // element fields of the next layer and the owned node's mass of the next
     // plane, loaded one iteration ahead (see sweep_tile)
     float pq_pre[3] = {0.f, 0.f, 0.f};        // p, q, ss
@@ -255,7 +260,7 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
         fetch_elem(k + 1);
         fetch_mass(k + 1);
 
-        float F[6];
+        double F[3];
         // float64 corner coordinates of component t from the LDS planes
         auto corner8 = [&](int t, double *X) {
 #pragma unroll
@@ -271,12 +276,17 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
                 x[c] = float(X[c] - X[0]);
             }
         };
+        auto modes8 = [](const float *x) {
+            return elem_modes(face_modes(x[0], x[1], x[2], x[3]),
+                              face_modes(x[4], x[5], x[6], x[7]));
+        };
 
-        // ---- stress: f = -sigma * node normal ----
+        // ---- stress and hourglass forces, in the element's modes ----
         if (compute) {
-            float x[8], y[8], z[8], pf[3][8];
+            ElemModes<float> xm, ym, zm;
             {
                 double X[8], Y[8], Z[8];
+                float x[8];
                 corner8(0, X);
                 corner8(1, Y);
                 corner8(2, Z);
@@ -287,111 +297,53 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
                     raise_error(s, -1);
                 }
                 local8(X, x);
-                local8(Y, y);
-                local8(Z, z);
+                xm = modes8(x);
+                local8(Y, x);
+                ym = modes8(x);
+                local8(Z, x);
+                zm = modes8(x);
             }
-            const float sig = -ep - eq;
-            node_normals(pf[0], pf[1], pf[2], x, y, z);
+            const float determ = float(evolo * ev);
+            ForceShape<float> sh;
+            force_shape(xm, ym, zm, frcp(determ), sh);
+            const float coef = hg * ess * float(emass) * frcp(fcbrt(determ));
+            const float press64 = (ep + eq) * 0.015625f;
 #pragma unroll
             for (int t = 0; t < 3; ++t) {
+                ElemModes<float> um;
+                {
+                    // no mode changes with a uniform velocity: the
+                    // velocities relative to corner 0
+                    double U[8];
+                    float u[8];
+                    corner8(3 + t, U);
+                    local8(U, u);
+                    um = modes8(u);
+                }
+                const float n1 = t == 0 ? sh.n[0].x : t == 1 ? sh.n[0].y : sh.n[0].z;
+                const float n2 = t == 0 ? sh.n[1].x : t == 1 ? sh.n[1].y : sh.n[1].z;
+                const float n3 = t == 0 ? sh.n[2].x : t == 1 ? sh.n[2].y : sh.n[2].z;
+                const ElemModes<float> Fm = force_modes(sh, n1, n2, n3, press64, coef, um);
+                const float face[2][4] = {
+                    {-Fm.a3, Fm.a1 - Fm.h2, Fm.a2 - Fm.h1, Fm.h3 - Fm.h4},
+                    {Fm.a3, Fm.a1 + Fm.h2, Fm.a2 + Fm.h1, Fm.h3 + Fm.h4}};
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    corner[t][c][tid] = -(sig * pf[t][c]);
+                for (int h = 0; h < 2; ++h) {
+                    const float ap = face[h][0] + face[h][1], am = face[h][0] - face[h][1];
+                    const float bp = face[h][2] + face[h][3], bm = face[h][2] - face[h][3];
+                    corner[t][4 * h][tid] = am - bm;
+                    corner[t][4 * h + 1][tid] = ap - bp;
+                    corner[t][4 * h + 2][tid] = ap + bp;
+                    corner[t][4 * h + 3][tid] = am + bm;
                 }
             }
         }
         fold(finalize, carry, layer, F, P);
 
-        // ---- hourglass control ----
-        if (hourglass) {
-            __builtin_amdgcn_s_setprio(0);
-            if (compute) {
-                const double vv = ev;
-                const float determ = float(evolo * vv);
-                const float volinv = frcp(determ);
-                float hourgam[8][4];
-                {
-                    float x[8], y[8], z[8];
-                    {
-                        double X[8];
-                        corner8(0, X);
-                        local8(X, x);
-                        corner8(1, X);
-                        local8(X, y);
-                        corner8(2, X);
-                        local8(X, z);
-                    }
-                    float hm[4][3];
-#pragma unroll
-                    for (int i1 = 0; i1 < 4; ++i1) {
-                        float hmx = x[0] * fb_gamma<float>(i1, 0);
-                        float hmy = y[0] * fb_gamma<float>(i1, 0);
-                        float hmz = z[0] * fb_gamma<float>(i1, 0);
-#pragma unroll
-                        for (int n = 1; n < 8; ++n) {
-                            hmx = hmx + x[n] * fb_gamma<float>(i1, n);
-                            hmy = hmy + y[n] * fb_gamma<float>(i1, n);
-                            hmz = hmz + z[n] * fb_gamma<float>(i1, n);
-                        }
-                        hm[i1][0] = hmx;
-                        hm[i1][1] = hmy;
-                        hm[i1][2] = hmz;
-                    }
-#pragma unroll
-                    for (int n = 0; n < 8; ++n) {
-                        const int *st = kStencil[n];
-                        float dvx, dvy, dvz;
-                        volu_der(x, y, z, st[0], st[1], st[2], st[3], st[4], st[5], dvx,
-                                 dvy, dvz);
-#pragma unroll
-                        for (int i1 = 0; i1 < 4; ++i1) {
-                            hourgam[n][i1] =
-                                fb_gamma<float>(i1, n) -
-                                volinv * (dvx * hm[i1][0] + dvy * hm[i1][1] + dvz * hm[i1][2]);
-                        }
-                    }
-                }
-                __builtin_amdgcn_s_setprio(1);
-                const float coefficient =
-                    hg * ess * float(emass) * frcp(fcbrt(determ));
-#pragma unroll
-                for (int t = 0; t < 3; ++t) {
-                    float u[8];
-                    {
-                        // the hourglass modes annihilate uniform velocities:
-                        // project the velocities relative to corner 0
-                        double U[8];
-                        corner8(3 + t, U);
-                        local8(U, u);
-                    }
-                    float h[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        h[i] = hourgam[0][i] * u[0] + hourgam[1][i] * u[1] +
-                               hourgam[2][i] * u[2] + hourgam[3][i] * u[3] +
-                               hourgam[4][i] * u[4] + hourgam[5][i] * u[5] +
-                               hourgam[6][i] * u[6] + hourgam[7][i] * u[7];
-                    }
-#pragma unroll
-                    for (int n = 0; n < 8; ++n) {
-                        corner[t][n][tid] =
-                            coefficient * (hourgam[n][0] * h[0] + hourgam[n][1] * h[1] +
-                                           hourgam[n][2] * h[2] + hourgam[n][3] * h[3]);
-                    }
-                }
-            }
-            fold(finalize, carry, layer, F + 3, P + 3);
-        }
-
         // ---- acceleration, symmetry planes, velocity, position: float64 ----
         __builtin_amdgcn_s_setprio(2);
         if (finalize) {
-            double fx = double(F[0]), fy = double(F[1]), fz = double(F[2]);
-            if (hourglass) {
-                fx += double(F[3]);
-                fy += double(F[4]);
-                fz += double(F[5]);
-            }
+            const double fx = F[0], fy = F[1], fz = F[2];
             const int n = (k * en + je) * en + ie;
             const double minv = 1.0 / nmass;
             double xdd = fx * minv;
