@@ -842,32 +842,30 @@ struct ElemU {
 
 // everything the element reads is loaded before any store, which the
 // compiler must assume may alias it: one wait for memory, not three
-__device__ __forceinline__ void load_elem_u(const DevFields &f, const DevMeshU &m, int par,
-                                            int el, ElemU &E)
+__device__ __forceinline__ void load_elem_u(const DevFields &f, int par, unsigned el,
+                                            const unsigned (&nodes)[8], ElemU &E)
 {
-    const int ne = f.num_elem;
-    int nodes[8];
+    const double *const x = parity_copy(f.x, par), *const y = parity_copy(f.y, par),
+                        *const z = parity_copy(f.z, par);
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-        nodes[c] = m.nodelist[c * ne + el];
+        E.x[c] = load_at(x, nodes[c]);
+        E.y[c] = load_at(y, nodes[c]);
+        E.z[c] = load_at(z, nodes[c]);
     }
+    E.p = load_at(f.p, el);
+    E.q = load_at(f.q, el);
+    E.v = load_at(f.v, el);
+    E.volo = load_at(f.volo, el);
+    E.ss = load_at(f.ss, el);
+    E.emass = load_at(f.elem_mass, el);
+    const double *const xd = parity_copy(f.xd, par), *const yd = parity_copy(f.yd, par),
+                        *const zd = parity_copy(f.zd, par);
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-        E.x[c] = f.x[par][nodes[c]];
-        E.y[c] = f.y[par][nodes[c]];
-        E.z[c] = f.z[par][nodes[c]];
-    }
-    E.p = f.p[el];
-    E.q = f.q[el];
-    E.v = f.v[el];
-    E.volo = f.volo[el];
-    E.ss = f.ss[el];
-    E.emass = f.elem_mass[el];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        E.vel[0][c] = f.xd[par][nodes[c]];
-        E.vel[1][c] = f.yd[par][nodes[c]];
-        E.vel[2][c] = f.zd[par][nodes[c]];
+        E.vel[0][c] = load_at(xd, nodes[c]);
+        E.vel[1][c] = load_at(yd, nodes[c]);
+        E.vel[2][c] = load_at(zd, nodes[c]);
     }
 }
 
@@ -1034,9 +1032,6 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
     if (blk >= b.num_blocks) {
         return;  // the whole block
     }
-    if (l == 0) {
-        start = start_cycle(from, s, prm.ic_mode, blk == 0);
-    }
     const int ne = f.num_elem;
     const int el = b.elem_start[blk] + l;
     const bool has = el < b.elem_start[blk + 1];
@@ -1057,6 +1052,10 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
     if (own) {
         cb = b.ncorner_start[node];
         ce = b.ncorner_start[node + 1];
+    }
+    // the lists are on their way before the scalars are waited for
+    if (l == 0) {
+        start = start_cycle(from, s, prm.ic_mode, blk == 0);
     }
     __syncthreads();
     if (!start.go) {
@@ -1186,6 +1185,22 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
     if (blk >= b.num_blocks) {
         return;  // the whole block
     }
+    const int ne = f.num_elem;
+    const int e0 = b.elem_start[blk];
+    const int el = e0 + l;
+    const bool has = el < b.elem_start[blk + 1];
+    const int node = b.node_start[blk] + l;
+    const bool own = node < b.node_start[blk + 1];
+    int slot[8];
+    unsigned nodes[8];
+    if (has) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            nodes[c] = unsigned(load_at(m.nodelist, unsigned(c * ne + el)));
+            slot[c] = load_at(m.corner_slot, unsigned(c * ne + el));
+        }
+    }
+    // the lists are on their way before the scalars are waited for
     if (l == 0) {
         start = start_cycle(from, s, prm.ic_mode, blk == 0);
     }
@@ -1193,22 +1208,11 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
     if (!start.go) {
         return;
     }
-    const int ne = f.num_elem;
-    const int par = start.par;
-    const double dt = start.dt;
-    const int e0 = b.elem_start[blk];
-    const int el = e0 + l;
-    const bool has = el < b.elem_start[blk + 1];
-    const int node = b.node_start[blk] + l;
-    const bool own = node < b.node_start[blk + 1];
-    int slot[8];
+    const int par = wave_uniform(start.par);
+    const double dt = wave_uniform(start.dt);
     ElemU E;
     if (has) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            slot[c] = m.corner_slot[c * ne + el];
-        }
-        load_elem_u(f, m, par, el, E);
+        load_elem_u(f, par, unsigned(el), nodes, E);
     }
     // the interior node's state is loaded with the element's (no other block
     // reads or moves it): its loads wait with the element's, not after the
