@@ -30,7 +30,7 @@ struct TransferItem {
 class FieldTransfer {
 public:
     static constexpr size_t kSlotBytes = size_t(4) << 20;
-    static constexpr int kSlots = 12;
+    static constexpr int kSlots = 8;
 
     ~FieldTransfer();
     hipError_t run(const TransferItem *items, int count, bool to_device, hipStream_t stream);
