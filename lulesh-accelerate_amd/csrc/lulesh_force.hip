@@ -1028,7 +1028,7 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
     constexpr int kN = kForceBlockElems;
     __shared__ double corner[3][8][kN];
     __shared__ CycleStart start;
-    const int blk = xcd_order(int(blockIdx.x), b.num_blocks), l = int(threadIdx.x);
+    const int blk = mesh_block(f.num_elem, b.num_blocks), l = int(threadIdx.x);
     if (blk >= b.num_blocks) {
         return;  // the whole block
     }
@@ -1181,7 +1181,7 @@ __global__ __launch_bounds__(kForceBlockElems) void k_forces_u_blocks(DevFields 
     constexpr int kN = kForceBlockElems;
     __shared__ double corner[3][8][kN];
     __shared__ CycleStart start;
-    const int blk = xcd_order(int(blockIdx.x), b.num_blocks), l = int(threadIdx.x);
+    const int blk = mesh_block(f.num_elem, b.num_blocks), l = int(threadIdx.x);
     if (blk >= b.num_blocks) {
         return;  // the whole block
     }
@@ -1300,7 +1300,7 @@ __global__ __launch_bounds__(256) void k_nodes_u(DevFields f, DevMeshU m, DevSca
     if (s->active == 0 || s->error != 0) {
         return;
     }
-    const int t = xcd_order(int(blockIdx.x), int(gridDim.x)) * int(blockDim.x) + int(threadIdx.x);
+    const int t = mesh_block(f.num_elem, int(gridDim.x)) * int(blockDim.x) + int(threadIdx.x);
     const int i = t / kLanes, q = t % kLanes, l = int(threadIdx.x);
     // a group lies in one wave and leaves whole: its lanes share i
     if (i >= count) {

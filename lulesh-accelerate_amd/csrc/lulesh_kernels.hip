@@ -1428,7 +1428,7 @@ __global__ __launch_bounds__(256) void k_kinematics_q_u(DevFields f, DevMeshU m,
     if (s->active == 0 || s->error != 0) {
         return;
     }
-    const int el = xcd_order(int(blockIdx.x), int(gridDim.x)) * int(blockDim.x) + int(threadIdx.x);
+    const int el = mesh_block(f.num_elem, int(gridDim.x)) * int(blockDim.x) + int(threadIdx.x);
     const int ne = f.num_elem;
     if (el < ne) {
         int nodes[8];
@@ -1452,7 +1452,7 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_u(DevFields f, DevMeshU m, Dev
     if (skip) {
         return;
     }
-    const int slot = xcd_order(int(blockIdx.x), int(gridDim.x)) * int(blockDim.x) + int(threadIdx.x);
+    const int slot = mesh_block(f.num_elem, int(gridDim.x)) * int(blockDim.x) + int(threadIdx.x);
     unsigned long long cand_c = as_bits(kBig), cand_h = as_bits(kBig);
     if (slot < f.num_elem) {
         const int el = f.eos_order[slot];
