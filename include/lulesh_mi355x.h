@@ -159,9 +159,11 @@ int lulesh_run(lulesh_domain *d, int *cycles_done);
 /* Float64 arithmetic with fused multiply-adds (no counterpart in the
  * reference, whose C code rounds every product and every sum): enable = 1
  * lets the element phases (stress, hourglass, kinematics, Q gradients,
- * limiter, EOS) fuse a * b + c into one rounding and take their quotients
- * through refined hardware reciprocals, which makes the 150^3 step about 14%
- * faster.  Results then differ from the reference by rounding only:
+ * limiter, EOS) fuse a * b + c into one rounding, form forces and kinematics in
+ * an element's modes and take their quotients through refined hardware
+ * reciprocals: 0.354 instead of 0.545 ms a cycle at 150^3.  The intermediate
+ * fields delv, delv_* and delx_* are stored by the last cycle of a call only,
+ * on domains beyond the last-level cache.  Results then differ from the reference by rounding only:
  * measured over full runs at 30^3 and 45^3, the same cycle counts, origin
  * energy within 1e-14 relative and fields within 1e-11 relative (the
  * accepted tolerance is 1e-10).  enable = 0, the default, rounds every value
