@@ -254,6 +254,10 @@ int launch(lulesh_domain *d, int kid, F &&body)
     return LULESH_OK;
 }
 
+// Whether the learned Q phase of n elements shares the repetitions of 64 over
+// a block (k_q_eos_dt_learned_nat has both sides measured).
+bool learned_small(int64_t n) { return n <= 50000; }
+
 int queue_cycle_u(lulesh_domain *d, const DevScalars *from, DevScalars *s)
 {
     // whole rounds over the XCDs (xcd_order)
@@ -354,10 +358,15 @@ int queue_cycle(lulesh_domain *d, int c, bool store)
              } else if (mixed) {
                  hipLaunchKernelGGL(k_q_eos_dt_mixed, dim3(ge), dim3(kBlock), 0, st, fm, s,
                                     p, d->eos_bands);
+             } else if (d->learned && learned_small(d->num_elem)) {
+                 hipLaunchKernelGGL(
+                     fused ? fused::k_q_eos_dt_learned_nat : k_q_eos_dt_learned_nat,
+                     dim3(unsigned((d->num_elem + 63) / 64)), dim3(kBlock), 0, st, f, s, p,
+                     d->learned, d->learned_z_max, d->learned_form);
              } else if (d->learned) {
                  hipLaunchKernelGGL(fused ? fused::k_q_eos_dt_learned : k_q_eos_dt_learned,
-                                    dim3(ge), dim3(kBlock), 0, st, f, s, p, d->learned,
-                                    d->learned_z_max, d->learned_form);
+                                    dim3(unsigned((d->num_elem + 63) / 64)), dim3(64), 0, st, f,
+                                    s, p, d->learned, d->learned_z_max, d->learned_form);
              } else if (d->eos_bands == 0) {
                  hipLaunchKernelGGL(fused ? fused::k_q_eos_dt_nat : k_q_eos_dt_nat, dim3(gq),
                                     dim3(kBlock), 0, st, f, s, p);

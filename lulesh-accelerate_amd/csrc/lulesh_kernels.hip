@@ -1339,32 +1339,20 @@ __global__ __launch_bounds__(256) void k_q_features(DevFields f, PhysParams prm,
     q[size_t(el) * 4 + 3] = qquad;
 }
 
-// k_q_eos_dt with the learned closure in place of the limiter: every wave
-// evaluates the network on its 64 elements on the matrix cores
-__global__ __launch_bounds__(256) void k_q_eos_dt_learned(DevFields f, DevScalars *s,
-                                                          PhysParams prm,
-                                                          const MlpFrags *net,
-                                                          float z_max, int form)
+namespace {
+
+// The Q terms of one wave's 64 elements with the learned closure in place of
+// the limiter, the network evaluated on the matrix cores; every lane of the
+// wave calls it (valid: the lane has an element).
+__device__ __forceinline__ void learned_q_wave(const DevFields &f, const PhysParams &prm,
+                                               const MlpFrags &F, float z_max, int form,
+                                               MlpWaveLds &L, int el, bool valid, QInputs &in,
+                                               double &qlin, double &qquad)
 {
-    __shared__ unsigned long long lds_c[4], lds_h[4];
-    __shared__ int skip;
-    __shared__ MlpWaveLds lds[4];
-    if (threadIdx.x == 0) {
-        skip = (s->active == 0 || s->error != 0) ? 1 : 0;
-    }
-    __syncthreads();
-    if (skip) {
-        return;
-    }
     const int lane = int(threadIdx.x) & 63;
-    MlpWaveLds &L = lds[threadIdx.x >> 6];
-    const MlpFrags &F = *net;
-    const int chunk = int(gridDim.x) - 1 - int(blockIdx.x);
-    const int slot = chunk * int(blockDim.x) + int(threadIdx.x);
-    const bool valid = slot < f.num_elem;
-    int el = 0, rep = 0;
-    QInputs in;
-    double qlin = 0.0, qquad = 0.0, ql_u = 0.0, qq_u = 0.0;
+    double ql_u = 0.0, qq_u = 0.0;
+    qlin = 0.0;
+    qquad = 0.0;
     bool use_net = false;
     float x[kMlpIn];
 #pragma unroll
@@ -1372,8 +1360,6 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_learned(DevFields f, DevScalar
         x[t] = 0.f;
     }
     if (valid) {
-        el = f.eos_order[slot];
-        rep = f.eos_rep[slot];
         int i, j, k;
         elem_ijk(f, el, i, j, k);
         q_inputs(f, prm, el, i, j, k, in);
@@ -1411,11 +1397,77 @@ __global__ __launch_bounds__(256) void k_q_eos_dt_learned(DevFields f, DevScalar
     } else if (valid && form != 0) {
         monotonic_q(prm, in, qlin, qquad);  // the fallback: the plain limiter
     }
+}
+
+}  // namespace
+
+// k_q_eos_dt with the learned closure, one wave per block (20 KB of LDS): four
+// to a block left a CU four waves, one to a block seven.  150^3 step 820 -> 788
+// us, 100^3 264 -> 246.
+__global__ __launch_bounds__(64) void k_q_eos_dt_learned(DevFields f, DevScalars *s,
+                                                         PhysParams prm, const MlpFrags *net,
+                                                         float z_max, int form)
+{
+    __shared__ unsigned long long lds_c[4], lds_h[4];
+    __shared__ MlpWaveLds L;
+    // one wave: its lanes see the same flags
+    if (s->active == 0 || s->error != 0) {
+        return;
+    }
+    const int slot = (int(gridDim.x) - 1 - int(blockIdx.x)) * 64 + int(threadIdx.x);
+    const bool valid = slot < f.num_elem;
+    int el = 0, rep = 0;
+    if (valid) {
+        el = f.eos_order[slot];
+        rep = f.eos_rep[slot];
+    }
+    QInputs in;
+    double qlin, qquad;
+    learned_q_wave(f, prm, *net, z_max, form, L, el, valid, in, qlin, qquad);
     unsigned long long cand_c = as_bits(kBig), cand_h = as_bits(kBig);
     if (valid) {
         eos_dt_elem(f, s, prm, el, rep, in, qlin, qquad, cand_c, cand_h);
     }
     fold_minima(s, cand_c, cand_h, lds_c, lds_h);
+}
+
+// The same for small domains, in mesh order, 64 elements per block, their
+// repetitions shared by its four waves as in k_q_eos_dt_nat: on a chip that
+// is not full the launch lasts as long as the 20 evaluations of one wave.
+// Steps in us with k_q_eos_dt_learned and with this: 10^3 31.4, 24.0; 33^3 37.9,
+// 32.0; 36^3 46.8, 41.1; 38^3 48.2, 48.5; 45^3 59.6, 63.4.
+__global__ __launch_bounds__(256) void k_q_eos_dt_learned_nat(DevFields f, DevScalars *s,
+                                                              PhysParams prm,
+                                                              const MlpFrags *net, float z_max,
+                                                              int form)
+{
+    __shared__ unsigned long long lds_c[4], lds_h[4];
+    __shared__ int skip;
+    __shared__ MlpWaveLds L;
+    __shared__ RepLds rep_lds;
+    if (threadIdx.x == 0) {
+        skip = (s->active == 0 || s->error != 0) ? 1 : 0;
+    }
+    __syncthreads();
+    if (skip) {
+        return;
+    }
+    const int el = int(blockIdx.x) * 64 + int(threadIdx.x);
+    const bool valid = int(threadIdx.x) < 64 && el < f.num_elem;
+    QInputs in;
+    EosIn a{1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int extra = 0;
+    if (wave_uniform(int(threadIdx.x) >> 6) == 0) {
+        double qlin, qquad;
+        learned_q_wave(f, prm, *net, z_max, form, L, el, valid, in, qlin, qquad);
+        if (valid) {
+            extra = int(f.rep[el]) - 1;
+            f.ql[el] = qlin;
+            f.qq[el] = qquad;
+            a = eos_prepare(s, prm, in, qlin, qquad);
+        }
+    }
+    eos_nat_block(f, s, prm, el, valid, in, a, extra, lds_c, lds_h, rep_lds);
 }
 
 // ---------------------------------------------------------------------------

@@ -667,6 +667,8 @@ struct MlpFrags;
 __global__ void k_q_features(DevFields f, PhysParams prm, int form, float *feat, double *q);
 __global__ void k_q_eos_dt_learned(DevFields f, DevScalars *s, PhysParams prm,
                                    const MlpFrags *net, float z_max, int form);
+__global__ void k_q_eos_dt_learned_nat(DevFields f, DevScalars *s, PhysParams prm,
+                                       const MlpFrags *net, float z_max, int form);
 
 // The mixed-precision phases (the time step kernels are shared).
 __global__ void k_kinematics_q_mixed(DevFieldsMixed f, DevScalars *s, PhysParams prm);
@@ -685,6 +687,8 @@ __global__ void k_q_eos_dt(DevFields f, DevScalars *s, PhysParams prm, int bands
 __global__ void k_q_eos_dt_nat(DevFields f, DevScalars *s, PhysParams prm);
 __global__ void k_q_eos_dt_learned(DevFields f, DevScalars *s, PhysParams prm,
                                    const MlpFrags *net, float z_max, int form);
+__global__ void k_q_eos_dt_learned_nat(DevFields f, DevScalars *s, PhysParams prm,
+                                       const MlpFrags *net, float z_max, int form);
 __global__ void k_device_math(int op, int n, const double *a, const double *b,
                               double *out);
 hipError_t launch_force_sweep(const SweepShape &shape, const DevFields &f,

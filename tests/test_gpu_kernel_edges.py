@@ -197,3 +197,24 @@ def test_plane_blocks_are_the_sweep(lulesh_gpu, nx, mode, hgcoef):
     assert bad == []
     a.close()
     b.close()
+
+
+# 36^3 the largest whose repetitions are shared, 37^3 one wave per block
+@pytest.mark.parametrize("nx", [1, 4, 5, 36, 37])
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("fused", [False, True])
+def test_learned_q_outside_its_range_is_the_limiter(lulesh_gpu, nx, form, fused):
+    """With no input in the network's range every element keeps the plain
+    limiter: the plain step, bit for bit, in the learned Q kernels."""
+    import learned_q
+    net, _ = learned_q.load(learned_q.NET_FILE if form == 0 else learned_q.NET_FILE_STANDIN)
+    a = lulesh_gpu.Domain(nx, fused=fused)
+    b = lulesh_gpu.Domain(nx, fused=fused)
+    b.set_learned_q(net, 1e-30, form=form)
+    assert a.step(20) == b.step(20)
+    bad = [f for f in NODE + ELEM if not np.array_equal(a.get(f), b.get(f))]
+    assert bad == []
+    sa, sb = a.stats(), b.stats()
+    assert (sa.time, sa.dtcourant, sa.dthydro) == (sb.time, sb.dtcourant, sb.dthydro)
+    a.close()
+    b.close()
