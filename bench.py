@@ -175,8 +175,7 @@ def bench_batched(lulesh_amd, plain_value: float) -> dict:
     b = lulesh_amd.Batch(nx, ef)
     t_build = time.perf_counter() - t0
     print(f"bench: ensemble built in {t_build:.1f} s", file=sys.stderr, flush=True)
-    # the default launch shape (the autotuner's pick on this ensemble, set
-    # in the library), no tuning at run time
+    # the default launch shape, no tuning at run time
     shape = b.shape()
     t0 = time.perf_counter()
     rc = b.run()

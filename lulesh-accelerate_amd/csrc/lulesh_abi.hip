@@ -37,7 +37,8 @@ enum KernelId {
 };
 
 const char *const kKernelNames[KID_COUNT] = {
-    "k_time_increment", "k_force_sweep", "k_kinematics_q", "k_q_eos_dt",
+    "k_time_increment",  // no launches: the force kernels start a cycle (start_cycle)
+    "k_force_sweep", "k_kinematics_q", "k_q_eos_dt",
     "k_dt_finish", "k_forces_u_blocks", "k_nodes_u",
 };
 
