@@ -262,11 +262,14 @@ __device__ __forceinline__ void sweep_tile(const Fields &f, const DevScalars *fr
     for (int t = 0; t < 3; ++t) {
         lo[t] = read_face(pos[kbeg & 1][t]);
     }
+    __syncthreads();  // plane kbeg + 2 goes to the slot of plane kbeg
     // Iteration k: the element layer between planes k and k + 1 (both in
     // LDS, plane k + 2 on its way), then the nodes of plane k.  Its one
     // barrier comes when the thread's share of plane k + 2 and of the face
-    // forces is staged; what it waits for is read before the next one, from
-    // slots that are written after that.
+    // forces is staged.  It overwrites the positions of plane k, read in the
+    // iteration before (of plane kbeg, before the loop), the velocities of
+    // plane k - 1 and the face forces of plane k - 2: all read before the
+    // barrier that it follows.
     for (int k = kbeg; k < klast; ++k) {
         // wave priority rises towards the barrier, as in the exact build's
         // sweep (148 -> 143 us)
