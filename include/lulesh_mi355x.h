@@ -161,9 +161,11 @@ int lulesh_run(lulesh_domain *d, int *cycles_done);
  * lets the element phases (stress, hourglass, kinematics, Q gradients,
  * limiter, EOS) fuse a * b + c into one rounding, form forces and kinematics in
  * an element's modes and take their quotients through refined hardware
- * reciprocals: 0.354 instead of 0.545 ms a cycle at 150^3.  The intermediate
- * fields delv, delv_* and delx_* are stored by the last cycle of a call only,
- * on domains beyond the last-level cache.  Results then differ from the reference by rounding only:
+ * reciprocals: 0.354 instead of 0.545 ms a cycle at 150^3.  On domains beyond
+ * the last-level cache the Q gradients (delv_*, delx_*) are stored by the last
+ * cycle of a call and after an error only, and a VolumeError of the new volumes
+ * leaves ql and qq of the failed cycle, not of the one before.
+ * Results then differ from the reference by rounding only:
  * measured over full runs at 30^3 and 45^3, the same cycle counts, origin
  * energy within 1e-14 relative and fields within 1e-11 relative (the
  * accepted tolerance is 1e-10).  enable = 0, the default, rounds every value

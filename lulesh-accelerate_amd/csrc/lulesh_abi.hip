@@ -299,8 +299,7 @@ int queue_cycle_u(lulesh_domain *d, const DevScalars *from, DevScalars *s)
 }
 
 // Cycle c of a call (start_cycle says what c decides).  store: whether the
-// fused cycle leaves the intermediate fields (delv, the Q gradients) in
-// memory: the last cycle of a call does.
+// fused cycle leaves the Q gradients in memory: the last cycle of a call does.
 int queue_cycle(lulesh_domain *d, int c, bool store)
 {
     const DevScalars *const from = d->s + (c & 1);
@@ -967,6 +966,14 @@ int lulesh_step(lulesh_domain *d, int ncycles, int *cycles_done)
         *cycles_done = after.cycle - before.cycle;
     }
     if (after.error != 0) {
+        if (after.unstored != 0) {  // the call's last kinematics left its Q gradients out
+            hipLaunchKernelGGL(fused::k_q_gradients,
+                               dim3(unsigned((d->num_elem + kBlock - 1) / kBlock)), dim3(kBlock),
+                               0, d->stream, d->f, d->s);
+            HIP_TRY(d, hipGetLastError());
+            after.unstored = 0;
+            if ((rc = write_scalars(d, after))) return rc;
+        }
         return fail(d, after.error,
                     after.error == LULESH_VOLUME_ERROR ? "VolumeError" : "QStopError");
     }

@@ -865,8 +865,10 @@ namespace {
 // formed again by 2 (TX + TY) of the threads, those of the layers below and
 // above it by every thread.  Out go vnew, the rate of volume change, the
 // characteristic length and the two Q terms, which k_eos_dt_nat reads beside
-// its own state; the other seven fields only where the cycle is one whose
-// fields a caller can read (`store`, or the run ends with it).
+// its own state, and delv; the six gradients only where the cycle is one whose
+// fields a caller can read (`store`, or the run ends with it).  Of a cycle
+// that turns out to be one because of an error, k_q_gradients forms them again
+// from the node copy that s->unstored names.
 //
 // At 150^3: 449 MB and 133 us here, 358 MB and 83 us for the EOS.  43 M vector
 // instructions, half of the time's issue; three waves per SIMD (168 VGPRs)
@@ -900,6 +902,9 @@ __device__ __forceinline__ void kinematics_limit_tile(const DevFields &f, DevSca
     const int i = i0 + tx, j = j0 + ty;
     const bool own = i < nx && j < nx;
     store = store || s->last != 0;
+    if (tid == 0) {
+        s->unstored = store ? 0 : 1 + par;  // every block the same
+    }
 
     constexpr int kSlots = (PN + NT - 1) / NT;
     unsigned gnode[kSlots];  // node of plane 0 in each slot, the nearest outside the domain
@@ -1071,8 +1076,8 @@ __device__ __forceinline__ void kinematics_limit_tile(const DevFields &f, DevSca
                 store_at(f.vnew, e, r.vnew);
                 store_at(f.vdov, e, r.vdov);
                 store_at(f.arealg, e, r.arealg);
+                store_at(f.delv, e, r.vnew - v_old_k);
                 if (store) {
-                    store_at(f.delv, e, r.vnew - v_old_k);
                     store_at(f.delv_xi, e, r.delv[0]);
                     store_at(f.delv_eta, e, r.delv[1]);
                     store_at(f.delv_zeta, e, r.delv[2]);
@@ -1138,6 +1143,43 @@ hipError_t launch_kinematics_limit(const DevFields &f, DevScalars *s, const Phys
     hipLaunchKernelGGL(k_kinematics_limit, dim3(unsigned((tiles + 7) / 8 * 8)),
                        dim3(kLimitTX * kLimitTY), 0, stream, f, s, prm, nz, store ? 1 : 0);
     return hipGetLastError();
+}
+
+// The Q gradients that k_kinematics_limit left out, by its functions and so to
+// the same bits.
+__global__ __launch_bounds__(256) void k_q_gradients(DevFields f, const DevScalars *s)
+{
+    const int el = int(blockIdx.x) * 256 + int(threadIdx.x);
+    if (s->unstored == 0 || el >= f.num_elem) {
+        return;
+    }
+    const int par = s->unstored - 1;
+    int i, j, k;
+    elem_ijk(f, el, i, j, k);
+    const int en = f.nx + 1, n0 = (k * en + j) * en + i;
+    const int at[8] = {n0, n0 + 1, n0 + en + 1, n0 + en, n0 + en * en, n0 + en * en + 1,
+                       n0 + en * en + en + 1, n0 + en * en + en};
+    const double *const in[6] = {f.x[par], f.y[par], f.z[par], f.xd[par], f.yd[par], f.zd[par]};
+    double xyz[3][8], vel[3][8];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            xyz[t][c] = in[t][at[c]];
+            vel[t][c] = in[3 + t][at[c]];
+        }
+    }
+    const ElemModes<double> mu = corner_modes(vel[0]), mv = corner_modes(vel[1]),
+                            mw = corner_modes(vel[2]);
+    const Vec3<double> u[3] = {{mu.a1, mv.a1, mw.a1}, {mu.a2, mv.a2, mw.a2}, {mu.a3, mv.a3, mw.a3}};
+    // the gradients do not depend on the time step
+    const ElemKinematics r = elem_kinematics(elem_shape(xyz), u, f.volo[el], 0.0);
+    f.delv_xi[el] = r.delv[0];
+    f.delv_eta[el] = r.delv[1];
+    f.delv_zeta[el] = r.delv[2];
+    f.delx_xi[el] = r.delx[0];
+    f.delx_eta[el] = r.delx[1];
+    f.delx_zeta[el] = r.delx[2];
 }
 
 // EOS, volume update and time constraints after k_kinematics_limit, as

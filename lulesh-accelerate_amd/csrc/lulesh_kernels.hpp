@@ -53,6 +53,9 @@ struct DevScalars {
     int dt_pending;  // the accumulators hold minima not yet applied
     int cur;         // copy of the node arrays holding the state
     int last;        // 1 when the run ends with this cycle
+    // 0: the Q gradients of the last kinematics are in memory; else one more
+    // than the copy of the node arrays to form them from (k_kinematics_limit)
+    int unstored;
 };
 
 // The Courant and hydro minima of a cycle are gathered in the accumulators
@@ -168,6 +171,7 @@ __device__ __forceinline__ CycleStart start_cycle(const DevScalars *from, DevSca
         s->dt_pending = t.dt_pending;
         s->cur = t.cur;
         s->last = t.last;
+        s->unstored = t.unstored;
         if (t.error != 0) {
             atomicCAS(&s->error, 0, t.error);
         }
@@ -695,10 +699,12 @@ hipError_t launch_force_sweep(const SweepShape &shape, const DevFields &f,
                               const DevScalars *from, DevScalars *s,
                               const PhysParams &prm, hipStream_t stream);
 // kinematics and the limiter in one sweep, and the EOS that follows it; store:
-// whether the cycle leaves its intermediate fields in memory
+// whether the cycle leaves its Q gradients in memory.  k_q_gradients stores those
+// that the last sweep left out (s->unstored).
 int kinematics_limit_columns(int nx);  // its blocks per chunk of layers
 hipError_t launch_kinematics_limit(const DevFields &f, DevScalars *s, const PhysParams &prm,
                                    int nz, bool store, hipStream_t stream);
+__global__ void k_q_gradients(DevFields f, const DevScalars *s);
 __global__ void k_eos_dt_nat(DevFields f, DevScalars *s, PhysParams prm);
 __global__ void k_kinematics_q_batch(const BatchMember *members,
                                      const BatchWork *work, PhysParams prm);
