@@ -328,7 +328,10 @@ int lulesh_batch_get_field(lulesh_batch *b, int member, int field,
 /* Launch shapes: the sweep shape (as lulesh_set_sweep_shape), the number of
  * persistent blocks of the sweep and of the element kernels (0: one block
  * per tile / chunk), and the cycles replayed per captured graph (0: no
- * graph, plain launches).  Results do not depend on any of them. */
+ * graph, plain launches).  Results do not depend on any of them.  By default
+ * the planes per block (nz) are planned for the members left, anew as members
+ * stop; lulesh_batch_get_shape gives those of now, and lulesh_batch_set_shape
+ * with them keeps the plan, with others ends it. */
 int lulesh_batch_set_shape(lulesh_batch *b, int tx, int ty, int nz, int waves,
                            int sweep_blocks, int elem_blocks,
                            int cycles_per_graph);
@@ -345,8 +348,10 @@ int lulesh_batch_set_fused_multiply_add(lulesh_batch *b, int enable);
 /* The autotuner: times trial_cycles cycles of each candidate launch shape
  * (plain launches after one warm-up cycle) from a saved copy of the state,
  * restores the state and keeps the fastest shape with the batch's cycles
- * per graph.  *best_ms (may be NULL) receives its milliseconds per cycle.
- * The default shape is its pick on the 64-member ensemble of nx 16..64. */
+ * per graph.  The shape the batch has is the first candidate; fixed planes per
+ * block replace planned ones only when they are 5% faster.  After an error the
+ * batch has its shape again.  *best_ms (may be NULL) receives the milliseconds
+ * per cycle of the shape kept. */
 int lulesh_batch_autotune(lulesh_batch *b, int trial_cycles, double *best_ms);
 
 /* Milliseconds between the HIP events around the last step/run call. */
