@@ -63,17 +63,24 @@ __device__ __forceinline__ void elem_ijk(const DevFieldsMixed &f, int el, int &i
 
 // ---------------------------------------------------------------------------
 // Force sweep: the tiling of sweep_tile (lulesh_force.hip), with an element's
-// stress and hourglass forces formed together in its modes
-// (lulesh_modal.hpp), in float32, and a node's eight corners summed in
-// float64.
+// stress and hourglass forces formed in its modes (lulesh_modal.hpp) in
+// float32, each kind by itself.  They meet in float64: added there, turned
+// into corner forces, staged and summed over a node's eight corners, the
+// layers' two faces as modes within the thread, as in the fused float64 sweep.
 //
 // Against the two kinds corner by corner, staged one after the other and
-// summed in float32: 120^3 step 193 -> 174 us, 150^3 373 -> 341, 91^3 97 -> 87
-// (per thread and layer 1187 instead of 1629 vector instructions, two
-// barriers instead of four in the staging).  Error against the float64 run
-// over nine domains of 20^3 to 200^3, 100 to 900 cycles: the run's time 0.79
-// and p 1.01 of what it was, in the geometric mean; summed in float32, 1.2 to
-// 1.3.
+// summed in float32: 120^3 step 193 -> 174 us, 150^3 373 -> 341, 91^3 97 -> 85
+// (per thread and layer 892 instead of 1629 vector instructions, two barriers
+// instead of six).  With the kinds added in float32 the times are the same
+// (120^3 173.5, 150^3 341.1, 91^3 84.6), but the small kind lost what an ulp of
+// the large one holds.  Errors against the float64 run, relative to the form
+// corner by corner, in the geometric mean over 76 runs of 30^3 to 130^3 to
+// t = 1e-2: origin energy 1.04 (added in float32 1.11), total energy 1.07
+// (1.06), x 0.93, xd 1.02, e 1.00 (1.10), p 1.00, q 0.92, v 1.02 (1.15), ss
+// 1.01; over 36 stretches of 84 to 920 cycles on 20^3 to 200^3: time 0.73
+// (0.93), origin energy 0.99 (1.22), x 0.74 (1.08), xd 0.80 (1.13), e 0.92
+// (1.13), p 0.77 (1.08), v 0.84 (1.06).  Single runs scatter by half.  120^3:
+// origin energy 2.4e-6 (6.6e-6; corner by corner 2.5e-6).
 // ---------------------------------------------------------------------------
 template <int TX, int TY>
 __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
@@ -85,7 +92,7 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
     constexpr int PX = TX + 1;
     constexpr int PN = (TX + 1) * (TY + 1);
     __shared__ double plane[2][6][PN];
-    __shared__ float corner[3][8][NT];
+    __shared__ double side[3][3][NT];  // forces on corners 1, 2, 3 of each thread's face
     __shared__ int s_go, s_par;
     __shared__ double s_dt;
 
@@ -117,18 +124,6 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
     const int je = j0 - 1 + ty;
     const bool col_valid = ie >= 0 && ie < nx && je >= 0 && je < nx;
     const bool owner = tx >= 1 && ty >= 1 && ie <= nx && je <= nx;
-    // corner slots of element columns outside the domain hold +0.0, so the
-    // fold adds four corners per layer without testing which elements exist
-    // (adding +0.0 to a sum started from +0.0 changes no bits)
-    if (!col_valid) {
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                corner[t][c][tid] = 0.0f;
-            }
-        }
-    }
     const float hg = prm.hgcoef > 0.0 ? float(-prm.hgcoef * 0.01) : 0.0f;
 
     constexpr int kSlots = (PN + NT - 1) / NT;
@@ -175,40 +170,10 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
             }
         }
     };
-    // wave priority rises as a barrier approaches, as in the float64 sweep:
-    // 2 in the folds, the nodal update and the plane store, 1 in the element
-    // arithmetic
-    auto fold = [&](bool finalize, bool carry, bool layer, double *F, double *P) {
-        __syncthreads();
-        __builtin_amdgcn_s_setprio(2);
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            if (finalize) {
-                double acc = P[t];
-                if (layer) {
-                    acc += double(corner[t][2][tid - TX - 1]);
-                    acc += double(corner[t][3][tid - TX]);
-                    acc += double(corner[t][1][tid - 1]);
-                    acc += double(corner[t][0][tid]);
-                }
-                F[t] = acc;
-            }
-            if (carry) {
-                double acc = 0.0;
-                acc += double(corner[t][6][tid - TX - 1]);
-                acc += double(corner[t][7][tid - TX]);
-                acc += double(corner[t][5][tid - 1]);
-                acc += double(corner[t][4][tid]);
-                P[t] = acc;
-            }
-        }
-        __syncthreads();
-    };
-
     const int base = ty * PX + tx;
     const int nodeoff[4] = {base, base + 1, base + PX + 1, base + PX};
 
-    double P[3] = {0.0, 0.0, 0.0};
+    double top[3][4] = {};  // forces on the face of plane k from the layer below, as modes
     // element fields of the next layer and the owned node's mass of the next
     // plane, loaded one iteration ahead (see sweep_tile)
     float pq_pre[3] = {0.f, 0.f, 0.f};        // p, q, ss
@@ -230,29 +195,44 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
             mass_pre = f.nodal_mass[(kk * en + je) * en + ie];
         }
     };
+    // float64 corner values of component t between planes lo and hi
+    auto corner8 = [&](int lo, int t, double *X) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            X[c] = plane[lo][t][nodeoff[c]];
+            X[c + 4] = plane[lo ^ 1][t][nodeoff[c]];
+        }
+    };
+    // their modes in float32: no mode changes with a uniform value, so they are
+    // taken relative to corner 0
+    auto modes8 = [](const double *X) {
+        float x[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            x[c] = float(X[c] - X[0]);
+        }
+        return elem_modes(face_modes(x[0], x[1], x[2], x[3]),
+                          face_modes(x[4], x[5], x[6], x[7]));
+    };
     const int kbeg = (kc0 > 0) ? kc0 - 1 : 0;
     fetch_elem(kbeg);
     fetch_mass(kbeg);
     fetch_plane(kbeg);
     store_plane(kbeg & 1);
-    if (kbeg < nx) {
-        fetch_plane(kbeg + 1);
+    fetch_plane(kbeg + 1);  // kbeg < nx
+    store_plane((kbeg + 1) & 1);
+    if (kbeg + 1 < nx && kbeg + 1 < kc1) {
+        fetch_plane(kbeg + 2);
     }
+    __syncthreads();
+    // Iteration k: the element layer between planes k and k + 1 (both in LDS,
+    // plane k + 2 on its way), then the nodes of plane k.  Wave priority rises
+    // towards a barrier, as in the float64 sweep.
     for (int k = kbeg; k < kc1; ++k) {
         const bool layer = k < nx;
-        __syncthreads();
-        if (layer) {
-            store_plane((k + 1) & 1);
-        }
-        __syncthreads();
-        if (layer && k + 1 < nx && k + 1 < kc1) {
-            fetch_plane(k + 2);
-        }
         __builtin_amdgcn_s_setprio(1);
         const int lo = k & 1;
-        const int hi = lo ^ 1;
         const bool finalize = owner && k >= kc0;
-        const bool carry = owner && layer && k + 1 < kc1;
         const bool compute = layer && col_valid;
         const float ep = pq_pre[0], eq = pq_pre[1], ess = pq_pre[2];
         const double ev = vm_pre[0], evolo = vm_pre[1], emass = vm_pre[2];
@@ -260,111 +240,111 @@ __device__ __forceinline__ void sweep_tile_mixed(const DevFieldsMixed &f,
         fetch_elem(k + 1);
         fetch_mass(k + 1);
 
-        double F[3];
-        // float64 corner coordinates of component t from the LDS planes
-        auto corner8 = [&](int t, double *X) {
+        // ---- stress and hourglass forces, in the element's modes ----
+        double face[3][4];  // on the face of plane k, both layers
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                X[c] = plane[lo][t][nodeoff[c]];
-                X[c + 4] = plane[hi][t][nodeoff[c]];
+                face[t][c] = top[t][c];
+                top[t][c] = 0.0;
             }
-        };
-        // float32 copy relative to corner 0
-        auto local8 = [&](const double *X, float *x) {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                x[c] = float(X[c] - X[0]);
-            }
-        };
-        auto modes8 = [](const float *x) {
-            return elem_modes(face_modes(x[0], x[1], x[2], x[3]),
-                              face_modes(x[4], x[5], x[6], x[7]));
-        };
-
-        // ---- stress and hourglass forces, in the element's modes ----
+        }
         if (compute) {
             ElemModes<float> xm, ym, zm;
             {
                 double X[8], Y[8], Z[8];
-                float x[8];
-                corner8(0, X);
-                corner8(1, Y);
-                corner8(2, Z);
+                corner8(lo, 0, X);
+                corner8(lo, 1, Y);
+                corner8(lo, 2, Z);
                 // VolumeError on the Jacobian volume, then on v, which the
                 // reference tests for every element before it looks at
                 // hgcoef (reference/C/LULESH-OMP.cc:1579-1584, :1540-1543)
                 if (jacobian_volume(X, Y, Z) <= 0.0 || ev <= 0.0) {
                     raise_error(s, -1);
                 }
-                local8(X, x);
-                xm = modes8(x);
-                local8(Y, x);
-                ym = modes8(x);
-                local8(Z, x);
-                zm = modes8(x);
+                xm = modes8(X);
+                ym = modes8(Y);
+                zm = modes8(Z);
             }
             const float determ = float(evolo * ev);
             ForceShape<float> sh;
             force_shape(xm, ym, zm, frcp(determ), sh);
             const float coef = hg * ess * float(emass) * frcp(fcbrt(determ));
-            const float press64 = (ep + eq) * 0.015625f;
+            const double press64 = (double(ep) + double(eq)) * 0.015625;
 #pragma unroll
             for (int t = 0; t < 3; ++t) {
-                ElemModes<float> um;
-                {
-                    // no mode changes with a uniform velocity: the
-                    // velocities relative to corner 0
-                    double U[8];
-                    float u[8];
-                    corner8(3 + t, U);
-                    local8(U, u);
-                    um = modes8(u);
-                }
-                const float n1 = t == 0 ? sh.n[0].x : t == 1 ? sh.n[0].y : sh.n[0].z;
-                const float n2 = t == 0 ? sh.n[1].x : t == 1 ? sh.n[1].y : sh.n[1].z;
-                const float n3 = t == 0 ? sh.n[2].x : t == 1 ? sh.n[2].y : sh.n[2].z;
-                const ElemModes<float> Fm = force_modes(sh, n1, n2, n3, press64, coef, um);
-                const float face[2][4] = {
-                    {-Fm.a3, Fm.a1 - Fm.h2, Fm.a2 - Fm.h1, Fm.h3 - Fm.h4},
-                    {Fm.a3, Fm.a1 + Fm.h2, Fm.a2 + Fm.h1, Fm.h3 + Fm.h4}};
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const float ap = face[h][0] + face[h][1], am = face[h][0] - face[h][1];
-                    const float bp = face[h][2] + face[h][3], bm = face[h][2] - face[h][3];
-                    corner[t][4 * h][tid] = am - bm;
-                    corner[t][4 * h + 1][tid] = ap - bp;
-                    corner[t][4 * h + 2][tid] = ap + bp;
-                    corner[t][4 * h + 3][tid] = am + bm;
-                }
+                double U[8];
+                corner8(lo, 3 + t, U);
+                // the hourglass forces; the stress joins them in float64
+                const ElemModes<float> h =
+                    force_modes(sh, 0.0f, 0.0f, 0.0f, 0.0f, coef, modes8(U));
+                const double n1 = t == 0 ? sh.n[0].x : t == 1 ? sh.n[0].y : sh.n[0].z;
+                const double n2 = t == 0 ? sh.n[1].x : t == 1 ? sh.n[1].y : sh.n[1].z;
+                const double n3 = t == 0 ? sh.n[2].x : t == 1 ? sh.n[2].y : sh.n[2].z;
+                const double a1 = fused_madd(press64, n1, double(h.a1));
+                const double a2 = fused_madd(press64, n2, double(h.a2));
+                const double a3 = fused_madd(press64, n3, double(h.a3));
+                const double h1 = h.h1, h2 = h.h2, h3 = h.h3, h4 = h.h4;
+                face[t][0] -= a3;
+                face[t][1] += a1 - h2;
+                face[t][2] += a2 - h1;
+                face[t][3] += h3 - h4;
+                top[t][0] = a3;
+                top[t][1] = a1 + h2;
+                top[t][2] = a2 + h1;
+                top[t][3] = h3 + h4;
             }
         }
-        fold(finalize, carry, layer, F, P);
-
-        // ---- acceleration, symmetry planes, velocity, position: float64 ----
         __builtin_amdgcn_s_setprio(2);
+        // corner 0 stays, corners 1, 2, 3 go to the threads whose node they are
+        double F[3], own[6];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const double ap = face[t][0] + face[t][1], am = face[t][0] - face[t][1];
+            const double bp = face[t][2] + face[t][3], bm = face[t][2] - face[t][3];
+            F[t] = am - bm;
+            side[t][0][tid] = ap - bp;
+            side[t][1][tid] = ap + bp;
+            side[t][2][tid] = am + bm;
+            own[t] = plane[lo][t][base];
+            own[3 + t] = plane[lo][3 + t][base];
+        }
+        __syncthreads();  // the faces are staged, plane k is read
+        // ---- acceleration, symmetry planes, velocity, position: float64 ----
         if (finalize) {
-            const double fx = F[0], fy = F[1], fz = F[2];
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                F[t] += (side[t][1][tid - TX - 1] + side[t][2][tid - TX]) + side[t][0][tid - 1];
+            }
             const int n = (k * en + je) * en + ie;
             const double minv = 1.0 / nmass;
-            double xdd = fx * minv;
-            double ydd = fy * minv;
-            double zdd = fz * minv;
+            double xdd = F[0] * minv;
+            double ydd = F[1] * minv;
+            double zdd = F[2] * minv;
             if (ie == 0) xdd = 0.0;
             if (je == 0) ydd = 0.0;
             if (k == 0) zdd = 0.0;
-            double xd = plane[lo][3][base] + xdd * dt;
+            double xd = own[3] + xdd * dt;
             if (fabs(xd) < prm.u_cut) xd = 0.0;
-            double yd = plane[lo][4][base] + ydd * dt;
+            double yd = own[4] + ydd * dt;
             if (fabs(yd) < prm.u_cut) yd = 0.0;
-            double zd = plane[lo][5][base] + zdd * dt;
+            double zd = own[5] + zdd * dt;
             if (fabs(zd) < prm.u_cut) zd = 0.0;
             f.xd[par][n] = xd;
             f.yd[par][n] = yd;
             f.zd[par][n] = zd;
-            f.x[par][n] = plane[lo][0][base] + xd * dt;
-            f.y[par][n] = plane[lo][1][base] + yd * dt;
-            f.z[par][n] = plane[lo][2][base] + zd * dt;
+            f.x[par][n] = own[0] + xd * dt;
+            f.y[par][n] = own[1] + yd * dt;
+            f.z[par][n] = own[2] + zd * dt;
         }
+        if (k + 1 < nx && k + 1 < kc1) {
+            store_plane(lo);  // plane k + 2
+            if (k + 2 < nx && k + 2 < kc1) {
+                fetch_plane(k + 3);
+            }
+        }
+        __syncthreads();  // plane k + 2 is in LDS, the faces are read
     }
 }
 
