@@ -95,3 +95,26 @@ def test_jacobian_turned_over_inside_a_call(lulesh_gpu, step):
     assert differing(a, b) == []
     a.close()
     b.close()
+
+
+def test_volume_turned_over_inside_a_call(lulesh_gpu):
+    """An error of the kinematics, in the sweep that limits as well: the same
+    code in the same cycle as from the separate kernels."""
+    en, h, cycles = NX + 1, 1.125 / NX, 6.5
+    a, b = pair(lulesh_gpu)
+    got = []
+    for d in (a, b):
+        st = d.download_state()
+        xd = np.zeros((en, en, en))
+        xd[:, :, NX // 2] = h / (cycles * 1e-7)  # a node plane overtakes the next
+        st.update(xd=xd.ravel(), e=np.zeros(d.num_elem), deltatime=1e-7)
+        d.set_parameter("dtfixed", 1e-7)
+        for name in ("qlc_monoq", "qqc_monoq", "hgcoef"):
+            d.set_parameter(name, 0.0)
+        d.upload_state(st)
+        got.append(d.step(20, raise_on_error=False))
+    assert got == [(lulesh_gpu.VOLUME_ERROR, 7)] * 2
+    for f in ("x", "xd", "e", "p", "q", "v", "ss"):
+        assert np.array_equal(a.get(f).view(np.uint64), b.get(f).view(np.uint64)), f
+    a.close()
+    b.close()
