@@ -242,19 +242,21 @@ void cut_work(lulesh_batch *b, bool all)
     order_eos_chunks(b, all);
 }
 
-// room for n entries in a device list that is about to be written
+// room for n entries in a device list that is about to be written; without
+// memory for it the list in use stays
 template <typename T>
 int make_room(lulesh_batch *b, T **list, size_t *room, size_t n)
 {
     if (n <= *room) {
         return LULESH_OK;
     }
-    BHIP_TRY(b, hipStreamSynchronize(b->stream));
+    T *larger = nullptr;
+    BHIP_TRY(b, hipMalloc(&larger, n * sizeof(T)));
+    const hipError_t e = hipStreamSynchronize(b->stream);
     if (*list) (void)hipFree(*list);
-    *list = nullptr;
-    *room = 0;
-    BHIP_TRY(b, hipMalloc(list, n * sizeof(T)));
+    *list = larger;
     *room = n;
+    BHIP_TRY(b, e);
     return LULESH_OK;
 }
 
