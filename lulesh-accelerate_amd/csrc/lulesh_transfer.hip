@@ -28,6 +28,17 @@ namespace {
 constexpr size_t kThreadedBytes = size_t(4) << 20;
 constexpr int kThreads = 8;
 
+// The fields of a state of middling size go straight to and from the caller's
+// memory as well: below kDirectField a copy to pageable memory has a fixed cost
+// above a slot's, and from kDirectBytes on the threads win.  Through slots and
+// straight, in ms: uploads 10^3 0.165 and 0.17, 14^3 0.245 and 0.225, 30^3 0.29
+// and 0.23, 45^3 0.51 and 0.355, 50^3 0.545 and 0.48, 60^3 0.72 and 0.72; a
+// domain's first download, which makes the slots, 10^3 0.18 and 0.22, 14^3 0.27
+// and 0.155, 30^3 0.33 and 0.27, 45^3 0.82 and 0.62; later ones 50^3 0.67 and
+// 0.9, 60^3 0.8 and 1.2.
+constexpr size_t kDirectField = size_t(16) << 10;
+constexpr size_t kDirectBytes = size_t(10) << 20;
+
 __global__ __launch_bounds__(256) void k_gather(const double *field, const int32_t *place,
                                                 double *out, int n)
 {
@@ -158,8 +169,9 @@ hipError_t FieldTransfer::move_all(const TransferItem *items, int count, bool to
                                    hipStream_t stream)
 {
     size_t bytes = 0, largest = 0;
-    bool placed = false;
+    bool placed = false, plain = true;
     for (int i = 0; i < count; ++i) {
+        plain = plain && !items[i].f32 && !items[i].place;
         const size_t b = size_t(items[i].n) * device_bytes(items[i]);
         bytes += b;
         largest = std::max(largest, b);
@@ -168,13 +180,20 @@ hipError_t FieldTransfer::move_all(const TransferItem *items, int count, bool to
     if (bytes == 0) {
         return hipStreamSynchronize(stream);
     }
-    if (count == 1 && bytes < kThreadedBytes && !items->f32 && !items->place) {
-        void *const host = items->host;
-        const hipError_t r =
-            to_device
-                ? hipMemcpyAsync(items->dev, host, bytes, hipMemcpyHostToDevice, stream)
-                : hipMemcpyAsync(host, items->dev, bytes, hipMemcpyDeviceToHost, stream);
-        return r != hipSuccess ? r : hipStreamSynchronize(stream);
+    const bool direct = plain && (count == 1 ? bytes < kThreadedBytes
+                                             : largest >= kDirectField && bytes < kDirectBytes);
+    if (direct) {
+        hipError_t r = hipSuccess;
+        for (int i = 0; i < count && r == hipSuccess; ++i) {
+            void *const host = items[i].host;
+            const size_t b = size_t(items[i].n) * sizeof(double);
+            r = to_device ? hipMemcpyAsync(items[i].dev, host, b, hipMemcpyHostToDevice, stream)
+                          : hipMemcpyAsync(host, items[i].dev, b, hipMemcpyDeviceToHost, stream);
+            // one by one: 18^3 0.16 ms, all queued before one wait 0.195
+            if (r == hipSuccess && !to_device) r = hipStreamSynchronize(stream);
+        }
+        const hipError_t end = hipStreamSynchronize(stream);
+        return r != hipSuccess ? r : end;
     }
     hipError_t err = reserve(largest, placed);
     if (err != hipSuccess) {
