@@ -161,7 +161,7 @@ int lulesh_run(lulesh_domain *d, int *cycles_done);
  * lets the element phases (stress, hourglass, kinematics, Q gradients,
  * limiter, EOS) fuse a * b + c into one rounding, form forces and kinematics in
  * an element's modes and take their quotients through refined hardware
- * reciprocals: 0.354 instead of 0.545 ms a cycle at 150^3.  On domains beyond
+ * reciprocals: 0.356 instead of 0.547 ms a cycle at 150^3.  On domains beyond
  * the last-level cache the Q gradients (delv_*, delx_*) are stored by the last
  * cycle of a call and after an error only, and a VolumeError of the new volumes
  * leaves ql and qq of the failed cycle, not of the one before.

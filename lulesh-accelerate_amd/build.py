@@ -6,8 +6,9 @@
 Both land next to this file so they travel with the source tree.  Device
 code is compiled without FMA contraction (the kernels reproduce the
 reference's rounding) and without packed-FP32 instructions; the element
-phases are compiled a second time with contraction (LULESH_FUSED, the
-fused-multiply-add mode of the float64 step).
+phases are compiled a second time with LULESH_FUSED, whose pragmas and
+explicit fma say where multiply-adds fuse (the fused-multiply-add mode of
+the float64 step).
 """
 from __future__ import annotations
 

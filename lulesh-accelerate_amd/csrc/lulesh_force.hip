@@ -60,7 +60,7 @@ constexpr int kStencil[8][6] = {{1, 2, 3, 4, 5, 7}, {2, 3, 0, 5, 6, 4},
 // modes (lulesh_modal.hpp).
 //
 // FP64 issue bounded the corner form (81.5 M VALU wave instructions, 230 us
-// at 150^3); the modal form issues 46.3 M and takes 143 us, now bounded by
+// at 150^3); the modal form issues 46.3 M and takes 141 us, now bounded by
 // its two waves per SIMD (244 VGPRs) waiting for each other and for LDS:
 // issue is 62% busy, and its 580 MB pass at 4.1 TB/s of the 5.7 a copy
 // reaches.  What makes up the rest of the difference:

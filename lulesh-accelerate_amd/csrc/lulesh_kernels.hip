@@ -870,7 +870,7 @@ namespace {
 // that turns out to be one because of an error, k_q_gradients forms them again
 // from the node copy that s->unstored names.
 //
-// At 150^3: 449 MB and 133 us here, 358 MB and 83 us for the EOS.  43 M vector
+// At 150^3: 475 MB and 135 us here, 358 MB and 83 us for the EOS.  41 M vector
 // instructions, half of the time's issue; three waves per SIMD (168 VGPRs)
 // wait for each other at the two barriers of a layer.  What did not help:
 // the next plane held in registers across a layer (two waves, 142 us, or

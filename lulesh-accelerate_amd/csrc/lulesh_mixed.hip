@@ -72,7 +72,7 @@ __device__ __forceinline__ void elem_ijk(const DevFieldsMixed &f, int el, int &i
 // summed in float32: 120^3 step 193 -> 174 us, 150^3 373 -> 341, 91^3 97 -> 85
 // (per thread and layer 892 instead of 1629 vector instructions, two barriers
 // instead of six).  With the kinds added in float32 the times are the same
-// (120^3 173.5, 150^3 341.1, 91^3 84.6), but the small kind lost what an ulp of
+// (120^3 173.5, 150^3 341.1, 91^3 84.6; 200^3 810 against 828), but the small kind lost what an ulp of
 // the large one holds.  Errors against the float64 run, relative to the form
 // corner by corner, in the geometric mean over 76 runs of 30^3 to 130^3 to
 // t = 1e-2: origin energy 1.04 (added in float32 1.11), total energy 1.07
